@@ -81,6 +81,35 @@ def test_gemm_random_blocks(tc, dev, oracle, qt):
     assert ok, worst
 
 
+# From 9 tokens Q2_K, Q3_K and IQ4_XS run on the matrix cores too: one token
+# past the batched path's 8, tile edges (32 / 64 / 128 tokens, 256 rows) and
+# remainders, an odd number of weight units, K split over workgroups with the
+# fixup launch ((200, 1000, 4096) and (130, 300, 5120)), on random block bytes.
+#
+# Random blocks give weights up to 2^-5 * 4064, so outputs that cancel lie
+# below the fp32 rounding of their terms. The integer sums are exact on both
+# sides; the fp32 sum of nb block values v_b and the at most 10 roundings that
+# form each differ from the exact value by at most (nb + 10) 2^-24 sum |v_b| <=
+# (nb + 10) 2^-24 |xq| . |w| on either side. (One wrong quant moves its output
+# by about 1 / (8 K) of |xq| . |w|, several times that.)
+@pytest.mark.parametrize("M,N,K", [(9, 64, 256), (8, 257, 768), (32, 256, 1024), (33, 77, 768), (64, 255, 512),
+                                   (65, 300, 2304), (128, 512, 1280), (129, 129, 256), (200, 1000, 4096),
+                                   (130, 300, 5120)])
+@pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ4_XS])
+def test_gemm_low_bit_mfma(tc, dev, oracle, qt, M, N, K):
+    rng = np.random.default_rng(M * 5 + N + K + qt)
+    w = random_blocks(qt, rng, N, K)
+    x = gaussian(rng, (M, K))
+    got = tc.gemm(qt, to_dev(w, dev), to_dev(x, dev), N, K).cpu().numpy()
+    ref = oracle.matmul(qt, w, x, N, K)
+    qs, d, _ = oracle.quantize_q8k(x.ravel())
+    xa = np.abs(qs.reshape(-1, 256).astype(np.float64) * d.reshape(-1, 1)).reshape(M, K)
+    wa = np.abs(oracle.dequant(qt, w, N, K).reshape(N, K).astype(np.float64))
+    bound = 1e-4 + 1e-3 * np.abs(ref) + 2 * (K // 256 + 10) * 2.0**-24 * (xa @ wa.T)
+    worst = (np.abs(got - ref) / bound).max()
+    assert worst <= 1, f"{NAMES[qt]} M={M} N={N} K={K}: worst err/bound {worst:.3g}"
+
+
 @pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ2_XS, IQ4_XS, IQ4_NL, Q5_0])
 def test_gemm_exact_batched_types(tc, dev, oracle, qt):
     rng = np.random.default_rng(5 + qt)

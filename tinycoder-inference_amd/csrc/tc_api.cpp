@@ -96,8 +96,9 @@ bool type_ok(int t) { return t == TC_Q8_0 || t == TC_Q5_0 || t == TC_IQ4_NL || t
 
 bool g_q8_gemm_enabled = true;
 
-// Weight types of the int8 MFMA prefill GEMM (the others run the decode
-// kernel over groups of 8 tokens).
+// Weight types that always run the int8 MFMA prefill GEMM (and the only ones
+// tc_gemm_noalloc takes). The others have the decode kernel over groups of 8
+// tokens behind the matrix-core kernel: see gemm_route_mfma.
 bool mfma_gemm_type(int t) {
     return t == TC_Q4_K || t == TC_Q5_K || t == TC_Q6_K || t == TC_IQ3_XXS || t == TC_IQ3_S || t == TC_IQ2_S || t == TC_Q8_0;
 }
@@ -239,13 +240,18 @@ int device_cu_count() {
     return d ? d->num_cu : 0;
 }
 
+// The MFMA kernels use 32-bit buffer offsets.
+bool gemm_mfma_addressable(int type, uint32_t S, uint32_t rows, uint32_t cols) {
+    return uint64_t(S) * cols < (uint64_t(1) << 32) &&
+           uint64_t(rows) * tc_row_bytes(type, cols) < (uint64_t(1) << 32);
+}
+
 // Shape limits of the MFMA prefill GEMM (the int8-activation K-quant and IQ
 // types and Q8_0; cols % 256 == 0).
 int gemm_mfma_check(int type, uint32_t S, uint32_t rows, uint32_t cols) {
     if (!mfma_gemm_type(type)) return fail(TC_E_UNSUPPORTED, "type %d has no MFMA GEMM", type);
     if (cols % 256) return fail(TC_E_UNSUPPORTED, "cols=%u is not a multiple of 256", cols);
-    // 32-bit buffer offsets in the MFMA kernels
-    if (uint64_t(S) * cols >= (uint64_t(1) << 32) || uint64_t(rows) * tc_row_bytes(type, cols) >= (uint64_t(1) << 32))
+    if (!gemm_mfma_addressable(type, S, rows, cols))
         return fail(TC_E_UNSUPPORTED, "activations or weights of 4 GiB or more");
     return TC_OK;
 }
@@ -287,6 +293,41 @@ int gemm_entry_check(int type, const void *w, const float *x, const float *out, 
 
 int fail_code(int code, const char *msg) { return fail(code, "%s", msg); }
 }  // namespace tc
+
+namespace {
+
+// The exact batched path (the reference's launchQGemm,
+// GpuGemvIQInt8.hpp:771-847): the decode kernel over token groups.
+int gemm_batched(Device *dev, int type, const void *w, const float *x, float *out, uint32_t seq_len, uint32_t rows,
+                 uint32_t cols, hipStream_t st) {
+    for (uint32_t s0 = 0; s0 < seq_len; s0 += 8) {
+        const int rc = run_gemv(dev, type, w, nullptr, x + size_t(s0) * cols, nullptr, out + size_t(s0) * rows, nullptr,
+                                0, nullptr, std::min(8u, seq_len - s0), rows, cols, st);
+        if (rc) return rc;
+    }
+    return TC_OK;
+}
+
+// Whether a product of one of the types that also have the batched path goes
+// to the matrix cores; its scratch is in place then. Up to 8 tokens the
+// batched path is one launch that reads the weights once (Q3_K 18944x3584, 8
+// tokens: 29 us against 45). It also keeps the calls that need more than 32-bit
+// offsets or than the memory left, and those under graph capture, which it
+// serves from less scratch or none (the MFMA path's could not grow there, and
+// its address would be held by the graph).
+bool gemm_route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
+    if (S <= 8 || !tc::prefill_type(type) || !tc::gemm_mfma_addressable(type, S, rows, cols)) return false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (st != nullptr && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone))
+        return false;
+    size_t act_bytes = 0;
+    const size_t ws = tc::gemm_mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
+    if (ensure(dev->act, dev->act_bytes, act_bytes) && ensure(dev->aux, dev->aux_bytes, ws)) return true;
+    (void)hipGetLastError();  // the failed allocation's
+    return false;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -421,16 +462,12 @@ int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_le
         cols = p.cols;
     }
     if (!mfma_gemm_type(type)) {
-        // Q2_K / Q3_K / IQ4_XS and the fp32-activation IQ2_XS / IQ4_NL / Q5_0:
-        // the exact batched path (the reference's launchQGemm,
-        // GpuGemvIQInt8.hpp:771-847) -- the decode kernel over token groups.
-        for (uint32_t s0 = 0; s0 < seq_len; s0 += 8) {
-            const uint32_t S = std::min(8u, seq_len - s0);
-            rc = run_gemv(dev, type, w, nullptr, x + size_t(s0) * cols, nullptr, out + size_t(s0) * rows, nullptr, 0,
-                          nullptr, S, rows, cols, st);
-            if (rc) return rc;
-        }
-        return TC_OK;
+        // Q2_K / Q3_K / IQ4_XS and the fp32-activation IQ2_XS / IQ4_NL / Q5_0
+        if (tc::gemv_max_tokens(type, cols) == 0)
+            return fail(TC_E_UNSUPPORTED, "cols=%u too wide for the decode kernel", cols);
+        if (!gemm_route_mfma(dev, type, seq_len, rows, cols, st))
+            return gemm_batched(dev, type, w, x, out, seq_len, rows, cols, st);
+        return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
     }
     if ((rc = tc::gemm_mfma_check(type, seq_len, rows, cols))) return rc;
     size_t act_bytes = 0;

@@ -143,6 +143,7 @@ hipError_t launch_router_select(const float *logits, uint32_t S, uint32_t E, uin
 
 // ---- host-side helpers shared by the entry-point files (tc_api.cpp) ----
 int device_cu_count();
+bool gemm_mfma_addressable(int type, uint32_t S, uint32_t rows, uint32_t cols);
 int gemm_mfma_check(int type, uint32_t S, uint32_t rows, uint32_t cols);
 size_t gemm_mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu, size_t *act_bytes);
 int gemm_mfma_into(int type, const void *w, const float *x, float *out, uint32_t S, uint32_t rows, uint32_t cols,

@@ -1,5 +1,5 @@
 // tc_prefill.hip -- prefill GEMM out[m][n] = W[n] . x[m] for Q4_K, Q5_K,
-// Q6_K, Q8_0, IQ3_XXS, IQ3_S and IQ2_S weights on the int8 matrix cores
+// Q6_K, Q8_0, Q2_K, Q3_K, IQ3_XXS, IQ3_S, IQ2_S and IQ4_XS weights on the int8 matrix cores
 // (v_mfma_i32_32x32x32_i8). The weights of a tile are converted once per
 // token tile of up to 128 tokens, in the registers of the lanes that feed
 // them to the MFMA.
@@ -31,6 +31,11 @@
 //    in LDS once per workgroup.
 //  * IQ2_S: as Q4_K (256 rows); its codebook (8-byte entries) in LDS, the
 //    signs applied in registers.
+//  * Q2_K, Q3_K, IQ4_XS: as Q4_K (256 rows); conversions at each type below.
+//    18944x3584 against the decode kernel over groups of 8 tokens, which
+//    reads and decodes the weights once per group: Q3_K M = 512 1661 -> 75
+//    us (934 TOPS), M = 2048 6671 -> 253 us (1098 TOPS); Q2_K 2065 -> 91 and
+//    8234 -> 311; IQ4_XS 1498 -> 117 and 5705 -> 406.
 //
 // Q4_K (reference dequantizeQ4_KBlock, GGMLDequantize.hpp:436-477): a weight
 // of sub-block s is w = d*sc_s*q - dmin*m_s with q in 0..15 and sc_s, m_s in
@@ -138,6 +143,23 @@ struct PfType<kIQ3_S> {
 template <>
 struct PfType<kIQ2_S> {
     static constexpr uint32_t PR = 256, TSPLIT = 1, UB = 112, XB = 0;
+};
+// Q3_K: the 110-byte unit in a 112-byte window, as IQ3_S.
+template <>
+struct PfType<kQ3_K> {
+    static constexpr uint32_t PR = 256, TSPLIT = 1, UB = 112, XB = 0;
+};
+// Q2_K: the 84-byte unit (4-byte aligned, so always at byte 0) as 6 chunks at
+// a 112-byte row stride (slot 6 unused).
+template <>
+struct PfType<kQ2_K> {
+    static constexpr uint32_t PR = 256, TSPLIT = 1, UB = 112, XB = 0;
+};
+// IQ4_XS: the 136-byte unit (8-byte aligned) as 9 chunks at a 144-byte row
+// stride (the last chunk's upper half is past the unit).
+template <>
+struct PfType<kIQ4_XS> {
+    static constexpr uint32_t PR = 256, TSPLIT = 1, UB = 144, XB = 0;
 };
 // Codebook types: IQ3_XXS / IQ3_S the sign-applied grid (entries x 16 sign
 // nibbles x 4 bytes), IQ2_S its 1024 8-byte entries as they are.
@@ -466,7 +488,7 @@ __device__ __forceinline__ void k_chain_combine(const ASet &as, uint32_t toff, c
 // top give C = sum_s e . x exactly; acc += d8 * (d * C).
 struct Q6Frag {
     v4i bh[8], bl[8];
-    float d;
+    float d, dm;  // (dm: Q2_K)
 };
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 
@@ -524,11 +546,20 @@ __device__ __forceinline__ void q6_conv(const Q6Raw &r, uint32_t g, int s, Q6Fra
     }
 }
 
-// The conversion with the first token block's MFMAs (after the MFMA pair of
+// How a type's int8 planes combine into a superblock's value:
+//  * kDigits: e = 128 hi + lo, C = 128 (hi chain) + (lo chain), acc += d8 * (d * C)
+//  * kSingle: e fits int8, one chain, acc += d8 * (d * C)
+//  * kMins: the weights and the mins as two chains, acc += d8 * (d * C - dm * Mn)
+enum { kDigits, kSingle, kMins };
+__host__ __device__ constexpr int pf_planes(int type) {
+    return type == kQ3_K ? kSingle : type == kQ2_K ? kMins : kDigits;
+}
+
+// The conversion with the first token block's MFMAs (after the MFMAs of
 // block s, the planes of block s + 2), then each further block's MFMAs with
 // the previous block's combination (as for Q4_K).
 // conv(s): the planes of 32-block s into f.bh[s], f.bl[s]
-template <typename Conv>
+template <int MODE, typename Conv>
 __device__ __forceinline__ void dig_convert_chain(Conv &&conv, Q6Frag &f, const ASet &as, uint32_t toff, v16i &ch,
                                                   v16i &cl) {
     auto aread = [&](int s) __attribute__((always_inline)) { return as_v4i(lds4(as.lds + (as.o[s] + toff))); };
@@ -543,14 +574,29 @@ __device__ __forceinline__ void dig_convert_chain(Conv &&conv, Q6Frag &f, const 
     for (int s = 0; s < 8; ++s) {
         if (s + 1 < 8) af[(s + 1) & 1] = aread(s + 1);
         ch = mfma(af[s & 1], f.bh[s], ch);
-        cl = mfma(af[s & 1], f.bl[s], cl);
+        if constexpr (MODE != kSingle) cl = mfma(af[s & 1], f.bl[s], cl);
         if (s + 2 < 8) conv(s + 2);
         __builtin_amdgcn_sched_barrier(0);
     }
 }
-__device__ __forceinline__ void q6_chain_combine(const ASet &as, uint32_t toff, const Q6Frag &f, uint32_t g,
-                                                 v16i &ch, v16i &cl, const float *d8, const v16i &c,
-                                                 float (&acc)[16]) {
+// One output's combination (c, mn: a finished block's C and, for kMins, Mn).
+template <int MODE>
+__device__ __forceinline__ float dig_value(const Q6Frag &f, int c, int mn) {
+    if constexpr (MODE == kMins)
+        return fmaf(f.d, float(c), -f.dm * float(mn));
+    else
+        return f.d * float(c);
+}
+// A finished block's chains as the C and Mn that the next call combines.
+template <int MODE>
+__device__ __forceinline__ void dig_fold(const v16i &ch, const v16i &cl, v16i &c, v16i &mn) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c[r] = MODE == kDigits ? (ch[r] << 7) + cl[r] : ch[r];
+    if constexpr (MODE == kMins) mn = cl;
+}
+template <int MODE>
+__device__ __forceinline__ void dig_chain_combine(const ASet &as, uint32_t toff, const Q6Frag &f, v16i &ch, v16i &cl,
+                                                  const float *d8, const v16i &c, const v16i &mn, float (&acc)[16]) {
     auto aread = [&](int s) __attribute__((always_inline)) { return as_v4i(lds4(as.lds + (as.o[s] + toff))); };
     float4 dv[4];
 #pragma unroll
@@ -564,24 +610,141 @@ __device__ __forceinline__ void q6_chain_combine(const ASet &as, uint32_t toff, 
     for (int s = 0; s < 8; ++s) {
         if (s + 1 < 8) af[(s + 1) & 1] = aread(s + 1);
         ch = mfma(af[s & 1], f.bh[s], ch);
-        cl = mfma(af[s & 1], f.bl[s], cl);
+        if constexpr (MODE != kSingle) cl = mfma(af[s & 1], f.bl[s], cl);
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int rr = 2 * s + e;
             const float4 dq = dv[rr >> 2];
             const float dd = (rr & 3) == 0 ? dq.x : (rr & 3) == 1 ? dq.y : (rr & 3) == 2 ? dq.z : dq.w;
-            acc[rr] = fmaf(dd, f.d * float(c[rr]), acc[rr]);
+            acc[rr] = fmaf(dd, dig_value<MODE>(f, c[rr], mn[rr]), acc[rr]);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
 }
-__device__ __forceinline__ void q6_combine(const float *d8, const Q6Frag &f, const v16i &c, float (&acc)[16]) {
+template <int MODE>
+__device__ __forceinline__ void dig_combine(const float *d8, const Q6Frag &f, const v16i &c, const v16i &mn,
+                                            float (&acc)[16]) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const float4 dv = *reinterpret_cast<const float4 *>(d8 + 8 * q);
         const float dd[4] = {dv.x, dv.y, dv.z, dv.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[4 * q + e] = fmaf(dd[e], f.d * float(c[4 * q + e]), acc[4 * q + e]);
+        for (int e = 0; e < 4; ++e)
+            acc[4 * q + e] = fmaf(dd[e], dig_value<MODE>(f, c[4 * q + e], mn[4 * q + e]), acc[4 * q + e]);
+    }
+}
+
+// ---- Q3_K: B operands of one superblock ------------------------------------
+// Reference dequantizeQ3_KBlock (GGMLDequantize.hpp:612-648): element
+// 128n + 32k + l has t = bits 2k, 2k + 1 of qs[32n + l] with bit 4n + k of
+// hmask[l] above them, and w = d * (sc - 32) * (t - 4), sc the 6-bit scale of
+// its 16 weights. (32 - sc) * (t - 4) is -128..124, an int8, so one MFMA
+// chain gives -C exactly and d is negated. The 8 products of one scale are two
+// dwords, from which one v_perm_b32 takes four weights' products by their t:
+// ~29 VALU instructions per 32-block (digit planes as Q6_K's would be ~70)
+// and 8 MFMAs per token block where the two-plane types have 16.
+struct Q3Raw {
+    u4 hm, q[2];
+    uint32_t sc[4];  // the 16 scales, as bytes
+    uint32_t d;
+};
+__device__ __forceinline__ void q3_read(Q3Raw &r, const unsigned char *win, uint32_t sh, uint32_t g) {
+    r.hm = q6_read16(win, 16 * g, sh);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) r.q[n] = q6_read16(win, 32 + 32 * n + 16 * g, sh);
+    const u4 c = lds4(win + 96);
+    const uint32_t s0 = __builtin_amdgcn_alignbyte(c.y, c.x, sh), s1 = __builtin_amdgcn_alignbyte(c.z, c.y, sh),
+                   hi = __builtin_amdgcn_alignbyte(c.w, c.z, sh);
+    r.sc[0] = (s0 & 0x0F0F0F0Fu) | ((hi & 0x03030303u) << 4);
+    r.sc[1] = (s1 & 0x0F0F0F0Fu) | (((hi >> 2) & 0x03030303u) << 4);
+    r.sc[2] = ((s0 >> 4) & 0x0F0F0F0Fu) | (((hi >> 4) & 0x03030303u) << 4);
+    r.sc[3] = ((s1 >> 4) & 0x0F0F0F0Fu) | (((hi >> 6) & 0x03030303u) << 4);
+    r.d = sh ? c.w >> 16 : c.w & 0xFFFFu;
+}
+__device__ __forceinline__ void q3_conv(const Q3Raw &r, uint32_t g, int s, Q6Frag &f) {
+    // the lane's scale 2s + g: in word s / 2, byte 2 (s % 2) + g
+    const short m = short(32 - int(__builtin_amdgcn_ubfe(r.sc[s >> 1], 8 * (2 * (s & 1) + g), 8)));
+    const s16x2 mm = {m, m};
+    auto table = [&](s16x2 even, s16x2 odd) __attribute__((always_inline)) {
+        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, mm * odd), __builtin_bit_cast(uint32_t, mm * even),
+                                     0x06020400u);
+    };
+    const uint32_t t0 = table(s16x2{-4, -2}, s16x2{-3, -1}), t1 = table(s16x2{0, 2}, s16x2{1, 3});
+    const u4 qv = r.q[s >> 2];
+    const uint32_t q[4] = {qv.x, qv.y, qv.z, qv.w}, hm[4] = {r.hm.x, r.hm.y, r.hm.z, r.hm.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t t = ((q[i] >> (2 * (s & 3))) & 0x03030303u) | (((hm[i] >> s) & 0x01010101u) << 2);
+        f.bh[s][i] = int(__builtin_amdgcn_perm(t1, t0, t));
+    }
+}
+
+// ---- Q2_K: B operands of one superblock ------------------------------------
+// Reference dequantizeQ2_KBlock (GGMLDequantize.hpp:550-590): element
+// 128n + 32k + l has q = bits 2k, 2k + 1 of qs[32n + l]; the scale byte of its
+// 16 weights holds sc (low nibble) and m: w = d * sc * q - dmin * m. sc * q
+// (<= 45) is one int8 plane (its 4 values in a dword, taken by v_perm_b32), m
+// against the same activations the other: both sums come out exactly.
+struct Q2Raw {
+    u4 sc, q[2];
+    uint32_t d;
+};
+__device__ __forceinline__ void q2_read(Q2Raw &r, const unsigned char *win, uint32_t g) {
+    r.sc = lds4(win);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) r.q[n] = lds4(win + 16 + 32 * n + 16 * g);
+    r.d = lds1(win + 80);
+}
+__device__ __forceinline__ void q2_conv(const Q2Raw &r, uint32_t g, int s, Q6Frag &f) {
+    const uint32_t scw[4] = {r.sc.x, r.sc.y, r.sc.z, r.sc.w};
+    const uint32_t b = __builtin_amdgcn_ubfe(scw[s >> 1], 8 * (2 * (s & 1) + g), 8);  // byte 2s + g
+    const uint32_t tab = uint32_t(pkmul(0x03020100u, (b & 15u) * 0x00010001u));
+    const int m = int((b >> 4) * 0x01010101u);
+    const u4 qv = r.q[s >> 2];
+    const uint32_t q[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        f.bh[s][i] = int(__builtin_amdgcn_perm(tab, tab, (q[i] >> (2 * (s & 3))) & 0x03030303u));
+        f.bl[s][i] = m;
+    }
+}
+
+// ---- IQ4_XS: B operands of one superblock ----------------------------------
+// Reference dequantizeIQ4_XSBlock (GGMLDequantize.hpp:1044-1080): 32-block ib
+// has 16 bytes of nibbles (low: elements 0-15, high: 16-31, so k-half g takes
+// nibble g of all 16) into a table of 16 int8 values, scale ls - 32 with ls =
+// nibble ib of scales_l and bits 2ib of scales_h above it. e = (ls - 32) *
+// value (|e| <= 4064) takes Q6_K's digits, from value + 128 (1..241) as a byte.
+struct I4Raw {
+    u4 q[8];
+    uint32_t h, sl;  // d and scales_h, scales_l
+};
+__device__ __forceinline__ void i4_read(I4Raw &r, const unsigned char *win) {
+    auto rd8 = [&](uint32_t o) __attribute__((always_inline)) { return *reinterpret_cast<const uint2 *>(win + o); };
+    const uint2 h = rd8(0);
+    r.h = h.x;
+    r.sl = h.y;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint2 a = rd8(8 + 16 * i), b = rd8(16 + 16 * i);
+        r.q[i] = u4{a.x, a.y, b.x, b.y};
+    }
+}
+__device__ __forceinline__ void i4_conv(const I4Raw &r, uint32_t g, int s, Q6Frag &f) {
+    const short k = short(int(((r.sl >> (4 * s)) & 15u) | (((r.h >> (16 + 2 * s)) & 3u) << 4)) - 32);
+    const s16x2 k2 = {k, k}, off = {short(-128 * k), short(-128 * k)};
+    const u4 qv = r.q[s];
+    const uint32_t q[4] = {qv.x, qv.y, qv.z, qv.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t nib = (q[i] >> (4 * g)) & 0x0F0F0F0Fu, low = nib & 0x07070707u;
+        const uint32_t lo8 = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, low);  // entries 0-7
+        const uint32_t hi8 = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, low);  // entries 8-15
+        const uint32_t v = __builtin_amdgcn_perm(hi8, lo8, ((nib >> 1) & 0x04040404u) | 0x03020100u);
+        uint32_t hi, lo;
+        q6_digits(v, k2, off, hi, lo);
+        f.bh[s][i] = int(hi);
+        f.bl[s][i] = int(lo);
     }
 }
 
@@ -979,10 +1142,14 @@ __device__ __forceinline__ void stage(const PfArgs &a, const uint8_t *W, uint32_
         const uint32_t c = 64 * k + ln, r = c / CPR, p = c - CPR * r;
         if constexpr (TYPE == kIQ3_XXS)  // the window from the unit's 4-byte-aligned start (slot 6: unused)
             lds_load16(wbase + 1024 * k, rw, (((n0 + r) * a.row_bytes + b * 98) & ~3u) + 16 * min(p, 5u));
-        else if constexpr (TYPE == kIQ3_S)
+        else if constexpr (TYPE == kIQ3_S || TYPE == kQ3_K)
             lds_load16(wbase + 1024 * k, rw, (((n0 + r) * a.row_bytes + b * 110) & ~3u) + 16 * p);
         else if constexpr (TYPE == kIQ2_S)  // (slot 6: unused)
             lds_load16(wbase + 1024 * k, rw, (((n0 + r) * a.row_bytes + b * 82) & ~3u) + 16 * min(p, 5u));
+        else if constexpr (TYPE == kQ2_K)  // (slot 6: unused)
+            lds_load16(wbase + 1024 * k, rw, (n0 + r) * a.row_bytes + b * 84 + 16 * min(p, 5u));
+        else if constexpr (TYPE == kIQ4_XS)
+            lds_load16(wbase + 1024 * k, rw, (n0 + r) * a.row_bytes + b * 136 + 16 * p);
         else if constexpr (TYPE == kQ6_K)  // (slot 14: unused)
             lds_load16(wbase + 1024 * k, rw, (((n0 + r) * a.row_bytes + b * 210) & ~3u) + 16 * min(p, 13u));
         else
@@ -1143,12 +1310,13 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         for (int r = 0; r < 16; ++r) c[(t + 1) & 1][r] = (ch[r] << CSH) + cl[r];
                     }
                 }
-            } else if constexpr (TYPE == kQ6_K || TYPE == kIQ2_S) {
+            } else if constexpr (TYPE == kQ6_K || TYPE == kIQ2_S || TYPE == kQ3_K || TYPE == kQ2_K || TYPE == kIQ4_XS) {
+                constexpr int MODE = pf_planes(TYPE);
                 Q6Frag f;
                 auto d8_t = [&](int t) __attribute__((always_inline)) {
                     return reinterpret_cast<const float *>(bb + L::D8) + 32 * (tg * NB + t) + 4 * g;
                 };
-                v16i c[2], ch, cl;
+                v16i c[2], mn[2], ch, cl;
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (TYPE == kQ6_K) {
                     const uint32_t sh = ((n0 + rl) * a.row_bytes + b * 210) & 3u;
@@ -1161,33 +1329,47 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         __syncthreads();
                         stage_next(b);
                     }
-                    dig_convert_chain([&](int s) __attribute__((always_inline)) { q6_conv(rr, g, s, f); }, f, as, 0u,
+                    dig_convert_chain<MODE>([&](int s) __attribute__((always_inline)) { q6_conv(rr, g, s, f); }, f, as, 0u,
                                       ch, cl);
                     f.d = h2f(sh ? rr.dw >> 16 : rr.dw & 0xFFFFu);
+                } else if constexpr (TYPE == kQ3_K) {
+                    Q3Raw rr;
+                    q3_read(rr, wb + rl * T::UB, ((n0 + rl) * a.row_bytes + b * 110) & 3u, g);
+                    f.d = -h2f(rr.d);
+                    dig_convert_chain<MODE>([&](int s) __attribute__((always_inline)) { q3_conv(rr, g, s, f); }, f,
+                                            as, 0u, ch, cl);
+                } else if constexpr (TYPE == kQ2_K) {
+                    Q2Raw rr;
+                    q2_read(rr, wb + rl * T::UB, g);
+                    f.d = h2f(rr.d & 0xFFFFu);
+                    f.dm = h2f(rr.d >> 16);
+                    dig_convert_chain<MODE>([&](int s) __attribute__((always_inline)) { q2_conv(rr, g, s, f); }, f,
+                                            as, 0u, ch, cl);
+                } else if constexpr (TYPE == kIQ4_XS) {
+                    I4Raw rr;
+                    i4_read(rr, wb + rl * T::UB);
+                    f.d = h2f(rr.h & 0xFFFFu);
+                    dig_convert_chain<MODE>([&](int s) __attribute__((always_inline)) { i4_conv(rr, g, s, f); }, f,
+                                            as, 0u, ch, cl);
                 } else {
                     static_assert(!L::SW, "IQ2_S: two weight stages");
                     const uint32_t sh = ((n0 + rl) * a.row_bytes + b * 82) & 3u;
                     I2Raw rr;
                     i2_read(rr, wb + rl * T::UB, sh, g);
                     const unsigned char *grid = lds + L::GRID;
-                    dig_convert_chain([&](int s) __attribute__((always_inline)) { i2_conv(rr, grid, g, s, f); }, f,
+                    dig_convert_chain<MODE>([&](int s) __attribute__((always_inline)) { i2_conv(rr, grid, g, s, f); }, f,
                                       as, 0u, ch, cl);
                     f.d = 0.125f * h2f(rr.d);  // (a power of two: exact)
                 }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) c[0][r] = (ch[r] << 7) + cl[r];
+                dig_fold<MODE>(ch, cl, c[0], mn[0]);
 #pragma unroll
                 for (int t = 0; t < NB; ++t) {
-                    if (t + 1 < NB) {
-                        q6_chain_combine(as, 8192u * (t + 1), f, g, ch, cl, d8_t(t), c[t & 1], acc[t]);
-                    } else {
-                        q6_combine(d8_t(t), f, c[t & 1], acc[t]);
-                    }
+                    if (t + 1 < NB)
+                        dig_chain_combine<MODE>(as, 8192u * (t + 1), f, ch, cl, d8_t(t), c[t & 1], mn[t & 1], acc[t]);
+                    else
+                        dig_combine<MODE>(d8_t(t), f, c[t & 1], mn[t & 1], acc[t]);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (t + 1 < NB) {
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) c[(t + 1) & 1][r] = (ch[r] << 7) + cl[r];
-                    }
+                    if (t + 1 < NB) dig_fold<MODE>(ch, cl, c[(t + 1) & 1], mn[(t + 1) & 1]);
                 }
             } else if constexpr (TYPE == kIQ3_XXS || TYPE == kIQ3_S) {
                 I3Frag f;
@@ -1435,7 +1617,8 @@ int pf_nt(int type, uint32_t M) {
                       PLds<kQ6_K, 4>::total <= 160 * 1024 &&
                       PLds<kQ4_K, 4>::total <= 160 * 1024 &&
                       PLds<kQ8_0, 4>::total <= 160 * 1024 && PLds<kQ8W, 4>::total <= 160 * 1024 &&
-                      PLds<kIQ2_S, 4>::total <= 160 * 1024,
+                      PLds<kIQ2_S, 4>::total <= 160 * 1024 && PLds<kQ3_K, 4>::total <= 160 * 1024 &&
+                      PLds<kQ2_K, 4>::total <= 160 * 1024 && PLds<kIQ4_XS, 4>::total <= 160 * 1024,
                   "LDS of one workgroup");
     const int nt = M <= 32 ? 1 : M <= 64 ? 2 : 4;
     return type == kQ8_0 ? std::max(nt, 2) : nt;
@@ -1537,11 +1720,20 @@ hipError_t pf_launch(const PfArgs &a, hipStream_t st) {
     return hipGetLastError();
 }
 
+template <int TYPE>
+hipError_t pf_launch_nt(int nt, const PfArgs &a, hipStream_t st) {
+    switch (nt) {
+        case 1: return pf_launch<TYPE, 1>(a, st);
+        case 2: return pf_launch<TYPE, 2>(a, st);
+        default: return pf_launch<TYPE, 4>(a, st);
+    }
+}
+
 }  // namespace
 
 bool prefill_type(int type) {
     return type == kQ4_K || type == kQ5_K || type == kQ6_K || type == kQ8_0 || type == kIQ3_XXS || type == kIQ3_S ||
-           type == kIQ2_S;
+           type == kIQ2_S || type == kQ3_K || type == kQ2_K || type == kIQ4_XS;
 }
 
 // Workspace: the per-tile arrival counters (256-byte rounded), then the
@@ -1588,45 +1780,16 @@ hipError_t launch_prefill(int type, const void *W, const ActView &act, float *ou
         if (g.wide) return pf_launch<kQ8W, 4>(a, st);
         return g.nt == 2 ? pf_launch<kQ8_0, 2>(a, st) : pf_launch<kQ8_0, 4>(a, st);
     }
-    if (type == kIQ3_XXS) {
-        switch (g.nt) {
-            case 1: return pf_launch<kIQ3_XXS, 1>(a, st);
-            case 2: return pf_launch<kIQ3_XXS, 2>(a, st);
-            default: return pf_launch<kIQ3_XXS, 4>(a, st);
-        }
-    }
-    if (type == kQ5_K) {
-        switch (g.nt) {
-            case 1: return pf_launch<kQ5_K, 1>(a, st);
-            case 2: return pf_launch<kQ5_K, 2>(a, st);
-            default: return pf_launch<kQ5_K, 4>(a, st);
-        }
-    }
-    if (type == kQ6_K) {
-        switch (g.nt) {
-            case 1: return pf_launch<kQ6_K, 1>(a, st);
-            case 2: return pf_launch<kQ6_K, 2>(a, st);
-            default: return pf_launch<kQ6_K, 4>(a, st);
-        }
-    }
-    if (type == kIQ2_S) {
-        switch (g.nt) {
-            case 1: return pf_launch<kIQ2_S, 1>(a, st);
-            case 2: return pf_launch<kIQ2_S, 2>(a, st);
-            default: return pf_launch<kIQ2_S, 4>(a, st);
-        }
-    }
-    if (type == kIQ3_S) {
-        switch (g.nt) {
-            case 1: return pf_launch<kIQ3_S, 1>(a, st);
-            case 2: return pf_launch<kIQ3_S, 2>(a, st);
-            default: return pf_launch<kIQ3_S, 4>(a, st);
-        }
-    }
-    switch (g.nt) {
-        case 1: return pf_launch<kQ4_K, 1>(a, st);
-        case 2: return pf_launch<kQ4_K, 2>(a, st);
-        default: return pf_launch<kQ4_K, 4>(a, st);
+    switch (type) {
+        case kQ2_K: return pf_launch_nt<kQ2_K>(g.nt, a, st);
+        case kQ3_K: return pf_launch_nt<kQ3_K>(g.nt, a, st);
+        case kQ5_K: return pf_launch_nt<kQ5_K>(g.nt, a, st);
+        case kQ6_K: return pf_launch_nt<kQ6_K>(g.nt, a, st);
+        case kIQ2_S: return pf_launch_nt<kIQ2_S>(g.nt, a, st);
+        case kIQ3_S: return pf_launch_nt<kIQ3_S>(g.nt, a, st);
+        case kIQ3_XXS: return pf_launch_nt<kIQ3_XXS>(g.nt, a, st);
+        case kIQ4_XS: return pf_launch_nt<kIQ4_XS>(g.nt, a, st);
+        default: return pf_launch_nt<kQ4_K>(g.nt, a, st);
     }
 }
 

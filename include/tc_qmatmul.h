@@ -93,8 +93,10 @@ int tc_gemv_dual(int type, const void *wg, const void *wu, const float *x, float
  * Replaces tinycoder::gpu::int8Gemm (include/Int8Gemm.hpp:57-59,
  * GemmDispatch.cu:595). Int8 MFMA for the types the reference's GEMM takes
  * (Q4_K, Q5_K, Q6_K, Q8_0, IQ3_XXS, IQ3_S, IQ2_S; GemmDispatch.cu:600-602)
- * and, from 9 tokens on, for Q2_K, Q3_K and IQ4_XS; the other types, and those
- * three under stream capture, run the decode kernel over groups of 8 tokens.
+ * and, from 9 tokens on, for Q2_K, Q3_K and IQ4_XS; bf16 MFMA on x split into
+ * three exact pieces, from 9 tokens on, for IQ2_XS, IQ4_NL and Q5_0. Up to 8
+ * tokens, and under stream capture, those six run the decode kernel over
+ * groups of 8 tokens.
  * blocks_per_row must equal cols / block_elems. */
 int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_len, uint32_t rows,
             uint32_t cols, uint32_t blocks_per_row, void *stream);

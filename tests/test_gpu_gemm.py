@@ -110,6 +110,50 @@ def test_gemm_low_bit_mfma(tc, dev, oracle, qt, M, N, K):
     assert worst <= 1, f"{NAMES[qt]} M={M} N={N} K={K}: worst err/bound {worst:.3g}"
 
 
+# The fp32-activation types on the bf16 matrix cores (x as three exact bf16
+# pieces): from 9 tokens, tile edges and remainders, an odd number of 74-byte
+# units, split tiles, a tile kept whole over 9 superblocks ((300, 7000, 2304):
+# more tiles than workgroups), activations over 12 orders of magnitude.
+# Every product is exact; the fp32 sums of K / 32 block sums, each of at
+# most 12 roundings, stay within (K / 32 + 12) 2^-24 |x| . |w| of the exact
+# value here and in the oracle.
+@pytest.mark.parametrize("M,N,K", [(9, 64, 256), (8, 257, 768), (32, 256, 1024), (33, 77, 768), (64, 255, 512),
+                                   (65, 300, 2304), (128, 512, 1280), (129, 129, 256), (200, 1000, 4096),
+                                   (300, 7000, 2304)])
+@pytest.mark.parametrize("qt", [IQ4_NL, Q5_0, IQ2_XS])
+def test_gemm_fp32_activations_mfma(tc, dev, oracle, qt, M, N, K):
+    rng = np.random.default_rng(M * 3 + N + K + qt)
+    w = random_blocks(qt, rng, N, K)
+    x = gaussian(rng, (M, K)) * (10.0 ** rng.uniform(-6, 6, (M, 1))).astype(np.float32)
+    got = tc.gemm(qt, to_dev(w, dev), to_dev(x, dev), N, K).cpu().numpy()
+    rows = np.arange(N) if M * N * K < 1 << 28 else tile_edges(N, 256, 16, rng)
+    wr = w.reshape(N, -1)[rows]
+    ref = oracle_matmul_par(oracle, qt, wr, x, len(rows), K)
+    wa = np.abs(oracle.dequant(qt, wr, len(rows), K).astype(np.float64))
+    bound = 2 * (K // 32 + 12) * 2.0**-24 * (np.abs(x.astype(np.float64)) @ wa.T)
+    worst = (np.abs(got[:, rows] - ref) / bound).max()
+    assert worst <= 1, f"{NAMES[qt]} M={M} N={N} K={K}: worst err/bound {worst:.3g}"
+
+
+# An infinite or NaN activation reaches its token's outputs and no other's.
+@pytest.mark.parametrize("qt", [IQ4_NL, Q5_0, IQ2_XS])
+def test_gemm_fp32_activations_nonfinite(tc, dev, oracle, qt):
+    rng = np.random.default_rng(qt)
+    M, N, K = 40, 96, 512
+    w = random_blocks(qt, rng, N, K)
+    x = gaussian(rng, (M, K))
+    clean = tc.gemm(qt, to_dev(w, dev), to_dev(x, dev), N, K).cpu().numpy()
+    bad = x.copy()
+    bad[3, 7], bad[5, 300] = np.inf, np.nan
+    got = tc.gemm(qt, to_dev(w, dev), to_dev(bad, dev), N, K).cpu().numpy()
+    wf = oracle.dequant(qt, w, N, K)
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(got[3], np.inf * wf[:, 7], equal_nan=True)
+    assert np.isnan(got[5]).all()
+    keep = [m for m in range(M) if m not in (3, 5)]
+    assert np.array_equal(got[keep], clean[keep])
+
+
 @pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ2_XS, IQ4_XS, IQ4_NL, Q5_0])
 def test_gemm_exact_batched_types(tc, dev, oracle, qt):
     rng = np.random.default_rng(5 + qt)

@@ -308,6 +308,13 @@ int gemm_batched(Device *dev, int type, const void *w, const float *x, float *ou
     return TC_OK;
 }
 
+// Tokens per launch of the fp32-activation MFMA kernel: the bf16 pieces take 6
+// bytes per value, so long prompts go in chunks of about 96 MB of pieces
+// (2048 tokens at 8192 columns).
+uint32_t gemm_f32_chunk(uint32_t cols) {
+    return std::max(256u, uint32_t((size_t(96) << 20) / (size_t(cols) * 6)) / 128 * 128);
+}
+
 // Whether a product of one of the types that also have the batched path goes
 // to the matrix cores; its scratch is in place then. Up to 8 tokens the
 // batched path is one launch that reads the weights once (Q3_K 18944x3584, 8
@@ -316,12 +323,20 @@ int gemm_batched(Device *dev, int type, const void *w, const float *x, float *ou
 // serves from less scratch or none (the MFMA path's could not grow there, and
 // its address would be held by the graph).
 bool gemm_route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
-    if (S <= 8 || !tc::prefill_type(type) || !tc::gemm_mfma_addressable(type, S, rows, cols)) return false;
+    const bool f32 = tc::prefill_f32_type(type);
+    if (S <= 8 || !(f32 || tc::prefill_type(type)) || !tc::gemm_mfma_addressable(type, S, rows, cols)) return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (st != nullptr && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone))
         return false;
-    size_t act_bytes = 0;
-    const size_t ws = tc::gemm_mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
+    size_t act_bytes = 0, ws = 0;
+    if (f32) {
+        const uint32_t n = std::min(S, gemm_f32_chunk(cols));
+        act_bytes = tc::prefill_f32_act_bytes(n, cols);
+        ws = tc::prefill_f32_workspace_bytes(n, rows, cols, dev->num_cu);
+        if (S % n) ws = std::max(ws, tc::prefill_f32_workspace_bytes(S % n, rows, cols, dev->num_cu));
+    } else {
+        ws = tc::gemm_mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
+    }
     if (ensure(dev->act, dev->act_bytes, act_bytes) && ensure(dev->aux, dev->aux_bytes, ws)) return true;
     (void)hipGetLastError();  // the failed allocation's
     return false;
@@ -467,6 +482,16 @@ int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_le
             return fail(TC_E_UNSUPPORTED, "cols=%u too wide for the decode kernel", cols);
         if (!gemm_route_mfma(dev, type, seq_len, rows, cols, st))
             return gemm_batched(dev, type, w, x, out, seq_len, rows, cols, st);
+        if (tc::prefill_f32_type(type)) {
+            const uint32_t chunk = gemm_f32_chunk(cols);
+            for (uint32_t s0 = 0; s0 < seq_len; s0 += chunk) {
+                const hipError_t e =
+                    tc::launch_prefill_f32(type, w, x + size_t(s0) * cols, out + size_t(s0) * rows,
+                                           std::min(chunk, seq_len - s0), rows, cols, dev->num_cu, dev->act, dev->aux, st);
+                if (e != hipSuccess) return hip_fail(e, "bf16 MFMA GEMM");
+            }
+            return TC_OK;
+        }
         return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
     }
     if ((rc = tc::gemm_mfma_check(type, seq_len, rows, cols))) return rc;

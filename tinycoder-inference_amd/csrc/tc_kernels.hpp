@@ -89,6 +89,16 @@ size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int
 hipError_t launch_prefill(int type, const void *W, const ActView &act, float *out, uint32_t M, uint32_t N,
                           uint32_t K, int num_cu, void *workspace, hipStream_t st);
 
+// Prefill GEMM for the types that take fp32 activations (tc_prefill_f32.hip;
+// IQ4_NL, Q5_0, IQ2_XS): x is split into bf16 pieces in `act`
+// (prefill_f32_act_bytes, below 4 GiB), `workspace` of
+// prefill_f32_workspace_bytes holds partial tiles.
+bool prefill_f32_type(int type);
+size_t prefill_f32_act_bytes(uint32_t M, uint32_t K);
+size_t prefill_f32_workspace_bytes(uint32_t M, uint32_t N, uint32_t K, int num_cu);
+hipError_t launch_prefill_f32(int type, const void *W, const float *x, float *out, uint32_t M, uint32_t N, uint32_t K,
+                              int num_cu, void *act, void *workspace, hipStream_t st);
+
 // Grouped (MoE) form over expert-sorted rows: out[i][n] = act row i . W[e(i)]
 // row n for the token tiles of mt (count *ntm, at most ntm_max; tiles of at
 // most `tile` rows, tile from prefill_grouped_tile). ctr: the arrival

@@ -402,6 +402,52 @@ def test_router_cfg5_vs_oracle(tc, dev, oracle, S):
     assert (_bits(wts.cpu().numpy()) == _bits(rwts)).all()
 
 
+@pytest.mark.parametrize("S,E,H", [(1, 1, 8), (1, 5, 33), (3, 128, 2304), (8, 256, 1000), (15, 128, 1024), (17, 255, 264),
+                                   (64, 128, 2048), (65, 127, 136), (70, 300, 260), (256, 128, 128), (257, 130, 640),
+                                   (300, 129, 1028)])
+def test_router_logits_blocks(tc, dev, oracle, S, E, H):
+    """The logits bit for bit over every block shape of the launch (1, 4, 16
+    outputs per half-wave, the tiled kernel), ragged tokens and rows, widths
+    with 8-column groups and single columns left, and blocks of inputs that
+    start at unaligned addresses."""
+    rng = np.random.default_rng(S * 1000 + E + H)
+    w = (rng.standard_normal((E, H)) * 0.03).astype(np.float32)
+    x = rng.standard_normal((S, H)).astype(np.float32)
+    ref = oracle.matmul_f32(w, x, E, H)
+    for off in (0, 1):
+        wd, xd = (to_dev(np.concatenate([np.zeros(off, np.float32), a.ravel()]), dev)[off:] for a in (w, x))
+        lg, _, _ = tc.moe_router(wd.view(E, H), xd.view(S, H), 1)
+        assert (_bits(lg.cpu().numpy()) == _bits(ref)).all(), off
+
+
+@pytest.mark.parametrize("E,K", [(1, 1), (8, 8), (60, 6), (64, 64), (65, 8), (128, 64), (128, 65), (256, 8), (257, 8),
+                                 (512, 10), (513, 8)])
+def test_router_selection_orders(tc, dev, oracle, E, K):
+    """Selections where the parallel evaluation applies and where it does not,
+    side by side in one call: distinct logits; ties inside the top K, at its
+    edge and below it; probabilities too small for an exact sum; underflow to
+    zero; infinities and NaN."""
+    rng = np.random.default_rng(E * 100 + K)
+    lg = rng.standard_normal((12, E)).astype(np.float32)
+    order = np.argsort(-lg, axis=1)
+    lg[1, order[1, : min(2, E)]] = lg[1, order[1, 0]]                # ties at the top
+    lg[2, order[2, K - 1 : K + 1]] = lg[2, order[2, K - 1]]          # at the edge
+    lg[3, order[3, K:]] = -3.0                                       # below it
+    lg[4] = 0.5                                                      # all equal
+    lg[5] *= 12.0                                                    # no exact sum
+    lg[6] *= 300.0                                                   # underflow
+    lg[7] = np.round(lg[7] * 4) / 4                                  # many ties
+    lg[8, 0] = np.inf
+    lg[9, E // 2] = -np.inf
+    lg[10] = -np.inf
+    rids, rwts = oracle.moe_route(lg, K)
+    ids, wts = tc.moe_select(to_dev(lg, dev), K)
+    ids, wts = ids.cpu().numpy(), wts.cpu().numpy()
+    finite = ~np.isnan(rwts)
+    assert (ids == rids).all()
+    assert (np.isnan(wts) == ~finite).all() and (_bits(wts)[finite] == _bits(rwts)[finite]).all()
+
+
 def test_router_feeds_moe_ffn(tc, dev, oracle):
     """Router on the device feeding the expert FFN with no host round trip:
     the ids and weights the FFN consumes are the oracle router's, and the

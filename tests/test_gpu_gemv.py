@@ -287,6 +287,41 @@ def test_encoder_bit_exact_vs_oracle(tc, dev, oracle, qt):
     assert (got == ref).all(), f"{NAMES[qt]}: first diff {np.argwhere(got != ref)[:4].ravel()}"
 
 
+@pytest.mark.parametrize("qt", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_encoder_wave_edges(tc, dev, oracle, qt):
+    """The wave-per-unit encoders: unit counts around the units of a wave and
+    a workgroup, blocks and inputs at odd addresses, and values whose quotients
+    fall on and next to half-integers, are tiny or huge; for Q4_K and Q5_K also
+    subnormal, infinite or NaN (where Q6_K and Q8_0 convert a non-finite
+    quotient to an integer, which C leaves open)."""
+    import torch
+    rng = np.random.default_rng(qt + 500)
+    x = gaussian(rng, (35, 256))
+    x[1] = np.round(x[1] * 8) / 8
+    x[2] = rng.integers(-31, 32, 256) * 0.5          # halves of a scale of 1
+    x[2, ::32] = 15.5
+    x[3] = np.nextafter(x[2], np.float32(100))
+    x[4] *= 1e-30
+    x[5] *= 1e30
+    if qt in (Q4_K, Q5_K):
+        x[6], x[12] = x[6] * 1e-38, x[12] * 1e37
+        x[6, 7], x[13, 8] = np.inf, -np.inf
+        x[7, 9] = np.nan
+    x[8], x[9] = np.abs(x[8]), -np.abs(x[9])
+    x[10, 32:] = 0.0
+    x[11] = -0.0
+    for n in (1, 3, 4, 5, 15, 16, 17, 35):
+        ref = oracle.encode(qt, x[:n])
+        got = tc.encode(qt, to_dev(x[:n], dev)).cpu().numpy()
+        assert (got == ref).all(), f"{NAMES[qt]} n={n}: first diff {np.argwhere(got != ref)[:4].ravel()}"
+    xo = torch.zeros(35 * 256 + 1, device=dev)
+    xo[1:] = to_dev(x.ravel(), dev)
+    out = torch.full((ref.size + 2,), 0xA5, dtype=torch.uint8, device=dev)
+    tc._check(tc.lib.tc_encode(qt, xo.data_ptr() + 4, out.data_ptr() + 1, 35, 256, tc._stream()))
+    got = out.cpu().numpy()
+    assert (got[1:-1] == ref).all() and got[0] == 0xA5 and got[-1] == 0xA5
+
+
 def test_q4k_encoder_golden(tc, dev, golden):
     got = tc.encode(Q4_K, to_dev(golden["enc_q4k_x"], dev)).cpu().numpy()
     assert (got.reshape(-1, 144) == golden["enc_q4k_out"]).all()

@@ -181,127 +181,232 @@ __device__ __forceinline__ float first_abs_max(const float *x, int n, float *ama
     return maxv;
 }
 
-// ---- weight encoders (one thread per 256-weight unit) ------------------------
+// ---- encoders of Q4_K, Q5_K, Q6_K and Q8_0 (one wave per 256-weight unit) -----
+// Lane l holds weights 4l .. 4l + 3, so a unit is one 1 KB load and its bytes
+// are stored as dwords; groups of 32 weights are 8 lanes, of 16 weights 4. One
+// thread per unit read 1 KB apart from its neighbours and kept the unit's
+// quants in scratch: 18944x3584 Q4_K 124 -> 83 us (3.7 TB/s), Q5_K 3365 -> 95,
+// Q6_K 703 -> 77, Q8_0 1601 -> 62 (5.5 TB/s). Bound by the VALU (the IEEE
+// divisions) for the K-quants, by memory for Q8_0.
 
-// Q4_K: the reference's quantizeQ4KBlock (src/cpp/core/GGMLQuantize.cpp:47-95).
-__device__ void enc_q4k(const float *x, uint8_t *out) {
-    float scale[8], minv[8];
-    uint8_t q[256];
-    float maxScale = 0.0f, maxMin = 0.0f;
-    for (int g = 0; g < 8; ++g) {
-        const float *xp = x + 32 * g;
-        float mn = 0.0f, mx = 0.0f;
-        for (int i = 0; i < 32; ++i) {
-            mn = xp[i] < mn ? xp[i] : mn;
-            mx = mx < xp[i] ? xp[i] : mx;
-        }
-        const float sc = __fdiv_rn(mx - mn, 15.0f);
-        scale[g] = sc;
-        minv[g] = -mn;
-        maxScale = maxScale < sc ? sc : maxScale;
-        maxMin = maxMin < minv[g] ? minv[g] : maxMin;
-        for (int i = 0; i < 32; ++i) {
-            int v = sc > 1e-30f ? int(rintf(__fdiv_rn(xp[i] - mn, sc))) : 0;
-            v = v < 0 ? 0 : (v > 15 ? 15 : v);
-            q[32 * g + i] = uint8_t(v);
-        }
-    }
-    const uint16_t hd = maxScale > 0.0f ? f2h_trunc_ref(__fdiv_rn(maxScale, 63.0f)) : 0;
-    const uint16_t hdm = maxMin > 0.0f ? f2h_trunc_ref(__fdiv_rn(maxMin, 63.0f)) : 0;
-    const float d = h2f(hd), dm = h2f(hdm);
-    uint8_t sc6[8], m6[8];
-    for (int g = 0; g < 8; ++g) {
-        const int s = d > 1e-30f ? int(rintf(__fdiv_rn(scale[g], d))) : 0;
-        const int m = dm > 1e-30f ? int(rintf(__fdiv_rn(minv[g], dm))) : 0;
-        sc6[g] = uint8_t(s < 0 ? 0 : (s > 63 ? 63 : s));
-        m6[g] = uint8_t(m < 0 ? 0 : (m > 63 ? 63 : m));
-    }
-    out[0] = uint8_t(hd);
-    out[1] = uint8_t(hd >> 8);
-    out[2] = uint8_t(hdm);
-    out[3] = uint8_t(hdm >> 8);
-    for (int j = 0; j < 4; ++j) {
-        out[4 + j] = uint8_t(sc6[j] | ((sc6[j + 4] >> 4) << 6));
-        out[8 + j] = uint8_t(m6[j] | ((m6[j + 4] >> 4) << 6));
-        out[12 + j] = uint8_t((sc6[j + 4] & 0x0F) | ((m6[j + 4] & 0x0F) << 4));
-    }
-    for (int i = 0; i < 128; ++i) {
-        const int g0 = 2 * (i >> 5), l = i & 31;
-        out[16 + i] = uint8_t(q[32 * g0 + l] | (q[32 * (g0 + 1) + l] << 4));
-    }
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+
+// (the unit's bytes may start anywhere)
+__device__ __forceinline__ void put4(uint8_t *p, uint32_t v) { __builtin_memcpy(p, &v, 4); }
+__device__ __forceinline__ void put2(uint8_t *p, uint32_t v) {
+    const uint16_t h = uint16_t(v);
+    __builtin_memcpy(p, &h, 2);
 }
 
-// Q5_K (this build's encoder; the reference ships none): per-32 affine scale
-// (max-min)/31 and min -min, fp16 (RNE) super-scales max/63, 6-bit sub-scales
-// and mins packed like Q4_K's, q = clamp(rne((x + dmin*m)/(d*sc)), 0, 31) with
-// the low nibbles in qs and the fifth bits in qh, as the reference decoder
-// reads them (include/GGMLDequantize.hpp:346-380).
-__device__ void enc_q5k(const float *x, uint8_t *out) {
-    float scale[8], minv[8];
-    float maxScale = 0.0f, maxMin = 0.0f;
-    for (int g = 0; g < 8; ++g) {
-        const float *xp = x + 32 * g;
-        float mn = 0.0f, mx = 0.0f;
-        for (int i = 0; i < 32; ++i) {
-            mn = xp[i] < mn ? xp[i] : mn;
-            mx = mx < xp[i] ? xp[i] : mx;
-        }
-        scale[g] = __fdiv_rn(mx - mn, 31.0f);
-        minv[g] = -mn;
-        maxScale = maxScale < scale[g] ? scale[g] : maxScale;
-        maxMin = maxMin < minv[g] ? minv[g] : maxMin;
+template <int MASK>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+    if constexpr (MASK == 8)
+        return dpp_move<0x128>(v);  // row_ror:8
+    else
+        return uint32_t(__shfl_xor(int(v), MASK));
+}
+// Largest / smallest over aligned groups of 8 lanes (fmaxf and fminf drop NaN
+// like the comparisons of the serial scan).
+template <typename Op>
+__device__ __forceinline__ float group8(float v, Op op) {
+    v = op(v, dpp_f<0xB1>(v));
+    v = op(v, dpp_f<0x4E>(v));
+    return op(v, dpp_f<0x141>(v));  // row_half_mirror
+}
+__device__ __forceinline__ float fmax2(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ float fmin2(float a, float b) { return fminf(a, b); }
+
+// rne(n[i] / d) as integers, four at once: by the reciprocal where that is
+// sure to round the same way. r = rne(1 / d) and the product are off by at
+// most 2^-23 relative, the IEEE quotient by 2^-24; below 128 (every caller
+// clamps within that) a product further than 6e-5 from a half-integer
+// therefore rounds as the quotient does. (Where d or 1 / d leaves the normal
+// range the quotient itself is taken.)
+__device__ __forceinline__ void div_round(const float (&n)[4], float d, int (&q)[4]) {
+    const float r = __fdiv_rn(1.0f, d);
+    bool slow = !(fabsf(d) > 1e-30f && fabsf(d) < 1e30f);
+    float p[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        p[i] = n[i] * r;
+        const float k = rintf(p[i]);
+        slow = slow || fabsf(fabsf(p[i] - k) - 0.5f) < 6e-5f;
+        q[i] = int(k);
     }
-    const uint16_t hd = maxScale > 0.0f ? f2h_rne(__fdiv_rn(maxScale, 63.0f)) : 0;
-    const uint16_t hdm = maxMin > 0.0f ? f2h_rne(__fdiv_rn(maxMin, 63.0f)) : 0;
-    const float d = h2f(hd), dm = h2f(hdm);
-    uint8_t sc6[8], m6[8];
-    for (int g = 0; g < 8; ++g) {
-        const int s = d > 0.0f ? int(rintf(__fdiv_rn(scale[g], d))) : 0;
-        const int m = dm > 0.0f ? int(rintf(__fdiv_rn(minv[g], dm))) : 0;
-        sc6[g] = uint8_t(s < 0 ? 0 : (s > 63 ? 63 : s));
-        m6[g] = uint8_t(m < 0 ? 0 : (m > 63 ? 63 : m));
+    if (slow) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = int(rintf(__fdiv_rn(n[i], d)));
     }
-    out[0] = uint8_t(hd);
-    out[1] = uint8_t(hd >> 8);
-    out[2] = uint8_t(hdm);
-    out[3] = uint8_t(hdm >> 8);
+}
+__device__ __forceinline__ uint32_t pack4(const int (&q)[4]) {
+    return uint32_t(q[0]) | (uint32_t(q[1]) << 8) | (uint32_t(q[2]) << 16) | (uint32_t(q[3]) << 24);
+}
+__device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
+// Header dword k (0: d and dmin, 1..3: the 6-bit scales and mins, packed in
+// get_scale_min_k4 order) of a Q4_K / Q5_K unit; h, six: d and the group's
+// scale in even lanes, dmin and the group's min in odd ones.
+__device__ __forceinline__ uint32_t kheader(uint32_t k, uint32_t h, uint32_t six) {
+    uint32_t w[4] = {uint32_t(__builtin_amdgcn_readlane(h, 0)) | (uint32_t(__builtin_amdgcn_readlane(h, 1)) << 16), 0, 0, 0};
+#pragma unroll
     for (int j = 0; j < 4; ++j) {
-        out[4 + j] = uint8_t(sc6[j] | ((sc6[j + 4] >> 4) << 6));
-        out[8 + j] = uint8_t(m6[j] | ((m6[j + 4] >> 4) << 6));
-        out[12 + j] = uint8_t((sc6[j + 4] & 0x0F) | ((m6[j + 4] & 0x0F) << 4));
+        const uint32_t sl = __builtin_amdgcn_readlane(six, 8 * j), sh = __builtin_amdgcn_readlane(six, 8 * j + 32);
+        const uint32_t ml = __builtin_amdgcn_readlane(six, 8 * j + 1), mh = __builtin_amdgcn_readlane(six, 8 * j + 33);
+        w[1] |= (sl | ((sh >> 4) << 6)) << (8 * j);
+        w[2] |= (ml | ((mh >> 4) << 6)) << (8 * j);
+        w[3] |= ((sh & 15u) | ((mh & 15u) << 4)) << (8 * j);
     }
-    uint8_t *qh = out + 16, *qs = out + 48;
-    for (int i = 0; i < 160; ++i) out[16 + i] = 0;
-    for (int g = 0; g < 8; ++g) {
-        const float es = d * float(sc6[g]), em = dm * float(m6[g]);
-        const int c = g >> 1, h = g & 1;
-        for (int l = 0; l < 32; ++l) {
-            int v = es > 0.0f ? int(rintf(__fdiv_rn(x[32 * g + l] + em, es))) : 0;
-            v = v < 0 ? 0 : (v > 31 ? 31 : v);
-            qs[32 * c + l] |= uint8_t((v & 15) << (4 * h));
-            qh[l] |= uint8_t((v >> 4) << (2 * c + h));
-        }
+    return k == 0 ? w[0] : k == 1 ? w[1] : k == 2 ? w[2] : w[3];
+}
+// Largest of the 8 groups' v over the lanes of the same parity, from 0 (within
+// a group, lanes of one parity hold the same value; NaN drops out).
+__device__ __forceinline__ float wave_max_parity(float v, uint32_t lane) {
+    v = fmaxf(fmaxf(v, 0.0f), dpp_f<0x128>(v));  // row_ror:8
+    auto at = [&](int l) __attribute__((always_inline)) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(uint32_t, v), l));
+    };
+    const float e = fmaxf(fmaxf(at(0), at(16)), fmaxf(at(32), at(48)));
+    const float o = fmaxf(fmaxf(at(1), at(17)), fmaxf(at(33), at(49)));
+    return (lane & 1) ? o : e;
+}
+
+// Q4_K: the reference's quantizeQ4KBlock (src/cpp/core/GGMLQuantize.cpp:47-95):
+// per 32 weights the affine fit scale = (max - min) / 15, min = -min (0 among
+// the candidates of both), 6-bit sub-scales against fp16 super-scales
+// maxScale / 63 and maxMin / 63 (truncated as its floatToHalf does).
+// Q5_K (this build's encoder; the reference ships none): the same with
+// (max - min) / 31, fp16 by rounding, and q = clamp(rne((x + dmin*m)/(d*sc)),
+// 0, 31) with the low nibbles in qs and the fifth bits in qh, as the reference
+// decoder reads them (include/GGMLDequantize.hpp:346-380).
+template <int TYPE>
+__device__ __forceinline__ void enc_wave_k(const float (&x)[4], uint32_t lane, uint8_t *out) {
+    constexpr bool Q5 = TYPE == kQ5_K;
+    const uint32_t g = lane >> 3, l = lane & 7;  // group, dword of its 32 weights
+    const float mn = group8(fminf(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])), 0.0f), fmin2);
+    const float mx = group8(fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), 0.0f), fmax2);
+    const float scale = __fdiv_rn(mx - mn, Q5 ? 31.0f : 15.0f), minv = -mn;
+    // even lanes: the scale of their group and the super-scale, odd lanes: the mins'
+    const float own = (lane & 1) ? minv : scale;
+    const float most = wave_max_parity(own, lane);
+    const uint32_t h = most > 0.0f ? uint32_t(Q5 ? f2h_rne(__fdiv_rn(most, 63.0f)) : f2h_trunc_ref(__fdiv_rn(most, 63.0f))) : 0u;
+    constexpr float least = Q5 ? 0.0f : 1e-30f;
+    const float d = h2f(h);
+    const int six = clampi(d > least ? int(rintf(__fdiv_rn(own, d))) : 0, 0, 63);
+    const float sub = d * float(six);  // (quad_perm [0,0,2,2] and [1,1,3,3]: the even and the odd lane's)
+    const float es = Q5 ? dpp_f<0xA0>(sub) : scale, em = Q5 ? dpp_f<0xF5>(sub) : -mn;
+    int q[4] = {0, 0, 0, 0};
+    if (es > least) {
+        // (Q4_K subtracts the min: x - mn is x + (-mn) exactly)
+        const float n[4] = {x[0] + em, x[1] + em, x[2] + em, x[3] + em};
+        div_round(n, es, q);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = clampi(q[i], 0, Q5 ? 31 : 15);
     }
+    const uint32_t v = pack4(q), low = v & 0x0F0F0F0Fu;
+    const uint32_t other = lane_xor<8>(low);  // group g ^ 1
+    const uint32_t hw = kheader(l & 3, h, uint32_t(six));
+    uint32_t qh = 0;
+    if constexpr (Q5) {
+        qh = ((v >> 4) & 0x01010101u) << g;
+        qh |= lane_xor<8>(qh);
+        qh |= lane_xor<16>(qh);
+        qh |= lane_xor<32>(qh);
+    }
+    constexpr uint32_t QS = Q5 ? 48 : 16;
+    if ((g & 1) == 0)
+        put4(out + QS + 16 * g + 4 * l, low | (other << 4));
+    else if (g == 1 && l < 4)
+        put4(out + 4 * l, hw);
+    else if (Q5 && g == 3)
+        put4(out + 16 + 4 * l, qh);
+}
+
+// Q6_K (this build's encoder; the reference ships none): per-16 group scale
+// m/-32 from the signed first-abs-max, block iscale = -128/M over the group
+// scales, int8 sub-scales, fp16 (RNE) d = 1/iscale, q = clamp(rne(x/(d*sc)),
+// -32, 31) + 32, packed as the reference decoder reads
+// (include/GGMLDequantize.hpp:503-527).
+__device__ __forceinline__ void enc_wave_q6k(const float (&x)[4], uint32_t lane, uint8_t *out) {
+    float xn[4];  // NaN of any kind as 0, which the scan for the largest |x| passes over alike
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xn[i] = x[i] == x[i] ? x[i] : 0.0f;
+    const float m = first_absmax<4>(xn, int(4 * (lane & 3)));
+    const float gs = m == 0.0f ? 0.0f : __fdiv_rn(m, -32.0f);
+    // the first group of largest |gs| (the lowest lane holding it)
+    const uint32_t ab = __builtin_bit_cast(uint32_t, fabsf(gs));
+    auto umax = [](uint32_t p, uint32_t q) { return p > q ? p : q; };
+    const uint32_t row = group_reduce<16>(ab, umax);
+    const uint32_t top = umax(umax(__builtin_amdgcn_readlane(row, 0), __builtin_amdgcn_readlane(row, 16)),
+                              umax(__builtin_amdgcn_readlane(row, 32), __builtin_amdgcn_readlane(row, 48)));
+    int q[4] = {32, 32, 32, 32};
+    int sc = 0;
+    uint32_t hd = 0;
+    if (top != 0) {
+        const uint32_t first = uint32_t(__builtin_ctzll(__ballot(ab == top)));
+        const float M = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(uint32_t, gs), first));
+        const float iscale = __fdiv_rn(-128.0f, M);
+        const int v = int(rintf(iscale * gs));
+        sc = int(int8_t(v > 127 ? 127 : v));
+        hd = f2h_rne(__fdiv_rn(1.0f, iscale));
+        const float dg = h2f(hd) * float(sc);
+        if (dg != 0.0f)
+            div_round(x, dg, q);
+        else
+            q[0] = q[1] = q[2] = q[3] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = clampi(q[i], -32, 31) + 32;
+    }
+    const uint32_t v = pack4(q), low = v & 0x0F0F0F0Fu;
+    const uint32_t half = lane >> 5, k = (lane >> 3) & 3, l = lane & 7;  // element 128 half + 32 k + 4 l
+    const uint32_t other = lane_xor<16>(low);                            // k ^ 2
+    uint32_t qh = ((v >> 4) & 0x03030303u) << (2 * k);
+    qh |= lane_xor<8>(qh);
+    qh |= lane_xor<16>(qh);
+    if (k < 2) put4(out + 64 * half + 32 * k + 4 * l, low | (other << 4));
+    if (k == 2) put4(out + 128 + 32 * half + 4 * l, qh);
+    if ((lane & 3) == 0) out[192 + (lane >> 2)] = uint8_t(sc);
+    if (lane == 63) put2(out + 208, hd);
 }
 
 // Q8_0 (8 blocks of 32): d = max|w|/127 as fp16 (RNE), q = rne(w/d), +-127.
-__device__ void enc_q8_0(const float *x, uint8_t *out) {
-    for (int b = 0; b < 8; ++b) {
-        const float *xb = x + 32 * b;
-        uint8_t *o = out + 34 * b;
-        float amax = 0.0f;
-        for (int i = 0; i < 32; ++i) amax = fabsf(xb[i]) > amax ? fabsf(xb[i]) : amax;
-        const uint16_t hd = f2h_rne(__fdiv_rn(amax, 127.0f));
-        const float d = h2f(hd);
-        o[0] = uint8_t(hd);
-        o[1] = uint8_t(hd >> 8);
-        for (int i = 0; i < 32; ++i) {
-            int q = d > 0.0f ? int(rintf(__fdiv_rn(xb[i], d))) : 0;
-            q = q < -127 ? -127 : (q > 127 ? 127 : q);
-            o[2 + i] = uint8_t(int8_t(q));
-        }
+__device__ __forceinline__ void enc_wave_q8_0(const float (&x)[4], uint32_t lane, uint8_t *out) {
+    const float amax = group8(fmaxf(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))), 0.0f), fmax2);
+    const uint32_t hd = f2h_rne(__fdiv_rn(amax, 127.0f));
+    const float d = h2f(hd);
+    int q[4] = {0, 0, 0, 0};
+    if (d > 0.0f) {
+        div_round(x, d, q);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = clampi(q[i], -127, 127) & 255;
+    }
+    uint8_t *o = out + 34 * (lane >> 3);
+    if ((lane & 7) == 0) put2(o, hd);
+    put4(o + 2 + 4 * (lane & 7), pack4(q));
+}
+
+constexpr int kEncUnits = 4;  // units per wave
+template <int TYPE, int U>
+__global__ __launch_bounds__(256) void k_encode_wave(const float *__restrict__ x, uint8_t *__restrict__ out,
+                                                     uint32_t nunits) {
+    // U consecutive units per wave, their loads issued first
+    const uint32_t u0 = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * U;
+    const uint32_t lane = threadIdx.x & 63;
+    f32x4 v[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+        if (u0 + i < nunits) v[i] = *reinterpret_cast<const f32x4_a4 *>(x + size_t(u0 + i) * 256 + 4 * lane);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        if (u0 + i >= nunits) break;  // wave-uniform
+        const float e[4] = {v[i][0], v[i][1], v[i][2], v[i][3]};
+        uint8_t *o = out + size_t(u0 + i) * unit_bytes(TYPE);
+        if constexpr (TYPE == kQ6_K) enc_wave_q6k(e, lane, o);
+        else if constexpr (TYPE == kQ8_0) enc_wave_q8_0(e, lane, o);
+        else enc_wave_k<TYPE>(e, lane, o);
     }
 }
+
+// ---- the other encoders (one thread per 256-weight unit) ---------------------
 
 // Q2_K (this build's encoder; the reference ships none): per-16 affine
 // scale (max-min)/3 and min -min (0 included in the range), fp16 (RNE)
@@ -395,56 +500,6 @@ __device__ void enc_q3k(const float *x, uint8_t *out) {
         const int n = e >> 7, j = (e >> 5) & 3, l = e & 31;
         out[32 + 32 * n + l] |= uint8_t((L[e] & 3) << (2 * j));
         out[l] |= uint8_t((L[e] >> 2) << (4 * n + j));
-    }
-}
-
-// Q6_K (this build's encoder; the reference ships none): per-16 group scale
-// m/-32 from the signed first-abs-max, block iscale = -128/M over the group
-// scales, int8 sub-scales, fp16 (RNE) d = 1/iscale, q = clamp(rne(x/(d*sc)),
-// -32, 31) + 32, packed as the reference decoder reads
-// (include/GGMLDequantize.hpp:503-527).
-__device__ void enc_q6k(const float *x, uint8_t *out) {
-    float gs[16];
-    for (int g = 0; g < 16; ++g) {
-        float amax;
-        const float m = first_abs_max(x + 16 * g, 16, &amax);
-        gs[g] = amax == 0.0f ? 0.0f : __fdiv_rn(m, -32.0f);
-    }
-    float amaxs;
-    const float M = first_abs_max(gs, 16, &amaxs);
-    for (int i = 0; i < 210; ++i) out[i] = 0;
-    uint8_t L[256];
-    if (amaxs == 0.0f) {
-        for (int e = 0; e < 256; ++e) L[e] = 32;
-    } else {
-        const float iscale = __fdiv_rn(-128.0f, M);
-        int8_t sc[16];
-        for (int g = 0; g < 16; ++g) {
-            const int v = int(rintf(iscale * gs[g]));
-            sc[g] = int8_t(v > 127 ? 127 : v);
-            out[192 + g] = uint8_t(sc[g]);
-        }
-        const uint16_t hd = f2h_rne(__fdiv_rn(1.0f, iscale));
-        out[208] = uint8_t(hd);
-        out[209] = uint8_t(hd >> 8);
-        const float dh = h2f(hd);
-        for (int e = 0; e < 256; ++e) {
-            const float dg = dh * float(sc[e >> 4]);
-            int q = dg != 0.0f ? int(rintf(__fdiv_rn(x[e], dg))) : 0;
-            q = q < -32 ? -32 : (q > 31 ? 31 : q);
-            L[e] = uint8_t(q + 32);
-        }
-    }
-    for (int half = 0; half < 2; ++half) {
-        uint8_t *ql = out + 64 * half;
-        uint8_t *qh = out + 128 + 32 * half;
-        const uint8_t *Lh = L + 128 * half;
-        for (int l = 0; l < 32; ++l) {
-            const int q1 = Lh[l], q2 = Lh[l + 32], q3 = Lh[l + 64], q4 = Lh[l + 96];
-            ql[l] = uint8_t((q1 & 0xF) | ((q3 & 0xF) << 4));
-            ql[l + 32] = uint8_t((q2 & 0xF) | ((q4 & 0xF) << 4));
-            qh[l] = uint8_t((q1 >> 4) | ((q2 >> 4) << 2) | ((q3 >> 4) << 4) | ((q4 >> 4) << 6));
-        }
     }
 }
 
@@ -789,8 +844,8 @@ __device__ void enc_iq2xs(const float *x, uint8_t *out) {
     }
 }
 
-// One kernel per weight type (one thread per 256-weight unit): kept apart so
-// that no kernel inlines every encoder.
+// One kernel per weight type (one thread per 256-weight unit; Q4_K, Q5_K, Q6_K
+// and Q8_0: k_encode_wave): kept apart so that no kernel inlines every encoder.
 template <int TYPE>
 __global__ __launch_bounds__(64) void k_encode(const float *__restrict__ x, uint8_t *__restrict__ out,
                                                uint32_t nunits) {
@@ -798,12 +853,8 @@ __global__ __launch_bounds__(64) void k_encode(const float *__restrict__ x, uint
     if (u >= nunits) return;
     const float *xu = x + size_t(u) * 256;
     uint8_t *o = out + size_t(u) * unit_bytes(TYPE);
-    if constexpr (TYPE == kQ4_K) enc_q4k(xu, o);
-    else if constexpr (TYPE == kQ8_0) enc_q8_0(xu, o);
-    else if constexpr (TYPE == kQ2_K) enc_q2k(xu, o);
+    if constexpr (TYPE == kQ2_K) enc_q2k(xu, o);
     else if constexpr (TYPE == kQ3_K) enc_q3k(xu, o);
-    else if constexpr (TYPE == kQ5_K) enc_q5k(xu, o);
-    else if constexpr (TYPE == kQ6_K) enc_q6k(xu, o);
     else if constexpr (TYPE == kIQ3_S) enc_iq3s(xu, o);
     else if constexpr (TYPE == kIQ2_S) enc_iq2s(xu, o);
     else if constexpr (TYPE == kIQ2_XS) enc_iq2xs(xu, o);
@@ -864,8 +915,11 @@ hipError_t launch_encode(int type, const float *x, void *out, uint32_t nunits, h
     switch (type) {
 #define TC_CASE(t) \
     case t: k_encode<t><<<g, 64, 0, st>>>(x, o, nunits); break;
-        TC_CASE(kQ4_K) TC_CASE(kQ8_0) TC_CASE(kQ2_K) TC_CASE(kQ3_K) TC_CASE(kQ5_K) TC_CASE(kQ6_K) TC_CASE(kIQ3_S)
-        TC_CASE(kIQ2_S) TC_CASE(kIQ2_XS) TC_CASE(kIQ4_XS) TC_CASE(kIQ4_NL) TC_CASE(kQ5_0) TC_CASE(kIQ3_XXS)
+        TC_CASE(kQ2_K) TC_CASE(kQ3_K) TC_CASE(kIQ3_S) TC_CASE(kIQ2_S) TC_CASE(kIQ2_XS) TC_CASE(kIQ4_XS) TC_CASE(kIQ4_NL) TC_CASE(kQ5_0) TC_CASE(kIQ3_XXS)
+#undef TC_CASE
+#define TC_CASE(t) \
+    case t: k_encode_wave<t, kEncUnits><<<uint32_t((uint64_t(nunits) + 4 * kEncUnits - 1) / (4 * kEncUnits)), 256, 0, st>>>(x, o, nunits); break;
+        TC_CASE(kQ4_K) TC_CASE(kQ5_K) TC_CASE(kQ6_K) TC_CASE(kQ8_0)
 #undef TC_CASE
         default: return hipErrorInvalidValue;
     }

@@ -96,8 +96,14 @@ __device__ __forceinline__ uint32_t quant4_sum(float4 v, float iscale, int *sum)
 // (lane l holds elements 4l..4l+3). Writes qs[0..255], *d and bsums[0..15],
 // and with dg the 32-wide sums s_p = bsums[2p] + bsums[2p + 1] as two exact
 // bf16 pieces: dg[p] = 128 * (s_p >> 7), dg[8 + p] = s_p & 127.
-__device__ __forceinline__ void quant_q8k_block_wave_v(float4 v, int8_t *qs, float *d, int16_t *bsums,
-                                                       uint16_t *dg = nullptr) {
+// A quantized block in the wave's registers: lane l's values 4l .. 4l + 3, the
+// sum of its group of 16, and the block's d.
+struct Q8KLane {
+    uint32_t packed;
+    int s16;
+    float d;
+};
+__device__ __forceinline__ Q8KLane quant_q8k_wave(float4 v) {
     const uint32_t lane = threadIdx.x & 63;
     const float e[4] = {v.x, v.y, v.z, v.w};
     const float maxv = first_absmax<64>(e, 4 * int(lane));
@@ -109,24 +115,32 @@ __device__ __forceinline__ void quant_q8k_block_wave_v(float4 v, int8_t *qs, flo
         packed = quant4_sum(v, iscale, &sum);
         dv = __fdiv_rn(1.0f, iscale);
     }
-    reinterpret_cast<uint32_t *>(qs)[lane] = packed;
-    const int s16 = quad_sum(sum);
-    if ((lane & 3) == 0) bsums[lane >> 2] = int16_t(s16);
-    if (lane == 0) *d = dv;
-    if (dg != nullptr) {
-        const int s32 = s16 + __shfl_xor(s16, 4);  // lanes 8p: bsums 2p and 2p+1
-        if ((lane & 7) == 0) {
-            // |s| <= 4064: 128 * (s >> 7) has at most 6 significant bits and
-            // s & 127 at most 7, so both are exact in bf16
-            dg[lane >> 3] = uint16_t(__builtin_bit_cast(uint32_t, float((s32 >> 7) * 128)) >> 16);
-            dg[8 + (lane >> 3)] = uint16_t(__builtin_bit_cast(uint32_t, float(s32 & 127)) >> 16);
-        }
-    }
+    return {packed, quad_sum(sum), dv};
+}
+// The two bf16 pieces of lane 8p's 32-wide sum s (bsums 2p and 2p + 1).
+// |s| <= 4064: 128 * (s >> 7) has at most 6 significant bits and s & 127 at
+// most 7, so both are exact in bf16.
+__device__ __forceinline__ void q8k_pieces(int s16, uint16_t &hi, uint16_t &lo) {
+    const int s32 = s16 + __shfl_xor(s16, 4);
+    hi = uint16_t(__builtin_bit_cast(uint32_t, float((s32 >> 7) * 128)) >> 16);
+    lo = uint16_t(__builtin_bit_cast(uint32_t, float(s32 & 127)) >> 16);
 }
 
-__device__ __forceinline__ void quant_q8k_block_wave(const float *x, int8_t *qs, float *d, int16_t *bsums,
-                                                     uint16_t *dg = nullptr) {
-    quant_q8k_block_wave_v(reinterpret_cast<const float4 *>(x)[threadIdx.x & 63], qs, d, bsums, dg);
+__device__ __forceinline__ void quant_q8k_block_wave_v(float4 v, int8_t *qs, float *d, int16_t *bsums,
+                                                       uint16_t *dg = nullptr) {
+    const uint32_t lane = threadIdx.x & 63;
+    const Q8KLane q = quant_q8k_wave(v);
+    reinterpret_cast<uint32_t *>(qs)[lane] = q.packed;
+    if ((lane & 3) == 0) bsums[lane >> 2] = int16_t(q.s16);
+    if (lane == 0) *d = q.d;
+    if (dg != nullptr) {
+        uint16_t hi, lo;
+        q8k_pieces(q.s16, hi, lo);
+        if ((lane & 7) == 0) {
+            dg[lane >> 3] = hi;
+            dg[8 + (lane >> 3)] = lo;
+        }
+    }
 }
 
 // Eight 32-element blocks by one full wave (8 lanes per block), lane values

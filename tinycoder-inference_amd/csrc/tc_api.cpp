@@ -600,7 +600,7 @@ int moe_grouped(Device *dev, const float *x, const int32_t *ids, const float *wt
         off += up(bytes);
         return o;
     };
-    const size_t o_pos = take(size_t(P) * 4), o_tok = take(size_t(P) * 4), o_mt = take(size_t(ntm_max) * 12),
+    const size_t o_pos = take(size_t(P) * 4), o_srt = take(size_t(P) * 4), o_mt = take(size_t(ntm_max) * 12),
                  o_ntm = take(4), o_g = take(size_t(P) * FF * 4), o_u = take(size_t(P) * FF * 4),
                  o_y = take(size_t(P) * H * 4), o_ax = take(LX.bytes + kGemmActSlack),
                  o_ah = take(LH.bytes + kGemmActSlack), o_ws = take(ws);
@@ -612,16 +612,16 @@ int moe_grouped(Device *dev, const float *x, const int32_t *ids, const float *wt
     if (!ensure(dev->aux, dev->aux_bytes, off)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", off);
     char *b = static_cast<char *>(dev->aux);
     int32_t *pos = reinterpret_cast<int32_t *>(b + o_pos);
-    uint32_t *tok = reinterpret_cast<uint32_t *>(b + o_tok), *mt = reinterpret_cast<uint32_t *>(b + o_mt);
+    uint32_t *srt = reinterpret_cast<uint32_t *>(b + o_srt), *mt = reinterpret_cast<uint32_t *>(b + o_mt);
     uint32_t *ntm = reinterpret_cast<uint32_t *>(b + o_ntm);
     float *g = reinterpret_cast<float *>(b + o_g), *u = reinterpret_cast<float *>(b + o_u);
     float *y = reinterpret_cast<float *>(b + o_y);
     const uint64_t gstride = uint64_t(FF) * (H / 256) * 144, dstride = uint64_t(H) * (FF / 256) * 144;
 
-    hipError_t e = tc::launch_moe_route(ids, P, top_k, E, 1, tile, pos, tok, mt, ntm, st);
+    hipError_t e = tc::launch_moe_route(ids, P, top_k, E, 1, tile, pos, srt, mt, ntm, st);
     if (e != hipSuccess) return hip_fail(e, "MoE router");
     uint32_t *ctr = reinterpret_cast<uint32_t *>(b + o_ctr);
-    e = tc::launch_quant_act_rows(x, tok, P, H, LX, b + o_ax, st, ctr, nctr);
+    e = tc::launch_quant_act_scatter(x, pos, T, top_k, H, LX, b + o_ax, st, ctr, nctr);
     if (e != hipSuccess) return hip_fail(e, "MoE activation gather");
     const tc::ActView ax = act_view(b + o_ax, LX, 0, TC_Q4_K, H);
     // gate and up in one launch (their tiles share the activations)

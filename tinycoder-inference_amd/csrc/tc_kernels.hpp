@@ -17,11 +17,13 @@ hipError_t launch_quant_act(int wtype, const float *x, uint32_t S, uint32_t cols
                             void *buf, hipStream_t st, bool block_major = false, uint32_t *zero = nullptr,
                             uint32_t nzero = 0);
 
-// Weight encoder: x[nunits][256] fp32 -> nunits units of `type`.
-// Q8_K block-major quantization of the gathered rows x[rows[s]], s < S.
-hipError_t launch_quant_act_rows(const float *x, const uint32_t *rows, uint32_t S, uint32_t cols, const ActLayout &L,
-                                 void *buf, hipStream_t st, uint32_t *zero = nullptr, uint32_t nzero = 0);
+// Q8_K block-major quantization of x[T][cols] into the T * top_k rows of L: row
+// pos[t * top_k + r] is token t (negative: none). No bsums.
+hipError_t launch_quant_act_scatter(const float *x, const int32_t *pos, uint32_t T, uint32_t top_k, uint32_t cols,
+                                    const ActLayout &L, void *buf, hipStream_t st, uint32_t *zero = nullptr,
+                                    uint32_t nzero = 0);
 
+// Weight encoder: x[nunits][256] fp32 -> nunits units of `type`.
 hipError_t launch_encode(int type, const float *x, void *out, uint32_t nunits, hipStream_t st);
 
 // rows x src_row_bytes -> rows x dst_row_bytes (a multiple of 4), each row
@@ -120,13 +122,12 @@ hipError_t launch_prefill_grouped(const void *W, uint64_t wstride, const ActView
 // Device-side router: pairs p = t*top_k + r (ids[p] in [0, E), others
 // skipped) sorted by expert; each expert's segment starts at a multiple of
 // `pad` rows and is cut into tiles of at most `tile` rows. pos[p] = the
-// pair's row (-1 for a skipped pair), row_tok[i] = the token of row i (~0 for
-// rows no pair lands on), mt = (row begin, row end, expert) per tile, *ntm =
-// the tile count. Sizes: moe_max_rows rows and moe_max_tiles tiles.
+// pair's row (-1 for a skipped pair), mt = (row begin, row end, expert) per
+// tile, *ntm = the tile count, scratch: a word per row
+// (npairs of them at pad 1). Size of mt: moe_max_tiles.
 uint32_t moe_max_tiles(uint32_t npairs, uint32_t n_experts, uint32_t tile);
-uint32_t moe_max_rows(uint32_t npairs, uint32_t n_experts, uint32_t pad);
 hipError_t launch_moe_route(const int32_t *ids, uint32_t npairs, uint32_t top_k, uint32_t n_experts, uint32_t pad,
-                            uint32_t tile, int32_t *pos, uint32_t *row_tok, uint32_t *mt, uint32_t *ntm,
+                            uint32_t tile, int32_t *pos, uint32_t *scratch, uint32_t *mt, uint32_t *ntm,
                             hipStream_t st);
 // h = silu(g) * u elementwise over nrows_max rows of ff values, written over g
 // (rows past the routed ones hold values nothing reads).

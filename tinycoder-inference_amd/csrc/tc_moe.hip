@@ -32,8 +32,7 @@ constexpr uint32_t kRouteLdsIds = 8192;    // ids read once into LDS up to this 
 // a token, count the earlier pairs of the segment instead.)
 __global__ __launch_bounds__(kRouteThreads) void k_moe_route(const int32_t *__restrict__ ids, uint32_t npairs,
                                                              uint32_t top_k, uint32_t E, uint32_t pad, uint32_t tile,
-                                                             uint32_t rows_max,
-                                                             int32_t *__restrict__ pos, uint32_t *__restrict__ row_tok,
+                                                             int32_t *__restrict__ pos, uint32_t *__restrict__ scratch,
                                                              uint32_t *__restrict__ mt, uint32_t *__restrict__ ntm) {
     __shared__ uint32_t cnt[kRouteMaxExperts], start[kRouteMaxExperts];
     __shared__ uint32_t bmap[kRouteMapWords], bpre[kRouteMapWords];
@@ -74,8 +73,6 @@ __global__ __launch_bounds__(kRouteThreads) void k_moe_route(const int32_t *__re
     if (use_map)
         for (uint32_t i = tid; i < E * W; i += kRouteThreads) bmap[i] = 0;
     if (tid == 0) dup = 0;
-    // rows that no pair lands on (padding, skipped pairs) are marked ~0
-    for (uint32_t i = tid; i < rows_max; i += kRouteThreads) row_tok[i] = ~0u;
     __syncthreads();
     for (uint32_t p = tid; p < npairs; p += kRouteThreads) {
         const int32_t e = eid[p];
@@ -131,7 +128,6 @@ __global__ __launch_bounds__(kRouteThreads) void k_moe_route(const int32_t *__re
         t0 += (c + tile - 1) / tile;
     }
     if (tid == kRouteThreads - 1) *ntm = t0;  // the last thread's end is the total
-    // (the row_tok marks above are ordered before the stores below by this barrier)
     __syncthreads();
     if (use_map && dup == 0) {
         // per expert, the earlier tokens' count at each bitmap word
@@ -149,16 +145,15 @@ __global__ __launch_bounds__(kRouteThreads) void k_moe_route(const int32_t *__re
             if (e >= 0 && uint32_t(e) < E) {
                 const uint32_t t = tok_of(p), i = uint32_t(e) * W + t / 32;
                 q = int32_t(start[e] + bpre[i] + __builtin_popcount(bmap[i] & ((1u << (t & 31)) - 1u)));
-                row_tok[q] = t;
             }
             pos[p] = q;
         }
     } else {
-        // the pair index at some row of its expert's segment (row_tok as
-        // scratch), then each pair's rank among the segment's pairs
+        // the pair index at some place of its expert's segment (unpadded),
+        // then each pair's rank among the segment's pairs
         for (uint32_t p = tid; p < npairs; p += kRouteThreads) {
             const int32_t e = eid[p];
-            if (e >= 0 && uint32_t(e) < E) row_tok[atomicAdd(&start[e], 1u)] = p;
+            if (e >= 0 && uint32_t(e) < E) scratch[atomicAdd(&start[e], 1u)] = p;
         }
         __syncthreads();
         for (uint32_t p = tid; p < npairs; p += kRouteThreads) {
@@ -167,15 +162,10 @@ __global__ __launch_bounds__(kRouteThreads) void k_moe_route(const int32_t *__re
             if (e >= 0 && uint32_t(e) < E) {
                 const uint32_t s1 = start[e], s0 = s1 - cnt[e];  // start[e] is now the segment's end
                 uint32_t rank = 0;
-                for (uint32_t r = s0; r < s1; ++r) rank += row_tok[r] < p ? 1u : 0u;
+                for (uint32_t r = s0; r < s1; ++r) rank += scratch[r] < p ? 1u : 0u;
                 q = int32_t(s0 + rank);
             }
             pos[p] = q;
-        }
-        __syncthreads();  // every scratch record read before row_tok is written
-        for (uint32_t p = tid; p < npairs; p += kRouteThreads) {
-            const int32_t q = pos[p];
-            if (q >= 0) row_tok[q] = p / top_k;
         }
     }
 }
@@ -255,18 +245,13 @@ uint32_t moe_max_tiles(uint32_t npairs, uint32_t n_experts, uint32_t tile) {
     return (npairs + tile - 1) / tile + std::min(npairs, n_experts);
 }
 
-uint32_t moe_max_rows(uint32_t npairs, uint32_t n_experts, uint32_t pad) {
-    return npairs + (pad - 1) * std::min(npairs, n_experts);
-}
-
 hipError_t launch_moe_route(const int32_t *ids, uint32_t npairs, uint32_t top_k, uint32_t n_experts, uint32_t pad,
-                            uint32_t tile, int32_t *pos, uint32_t *row_tok, uint32_t *mt, uint32_t *ntm,
+                            uint32_t tile, int32_t *pos, uint32_t *scratch, uint32_t *mt, uint32_t *ntm,
                             hipStream_t st) {
     if (npairs == 0 || top_k == 0 || n_experts == 0 || n_experts > kRouteMaxExperts || pad == 0 || tile == 0 ||
         uint64_t(npairs) * top_k >= (uint64_t(1) << 32))  // (the kernel's token-of-pair division)
         return hipErrorInvalidValue;
-    k_moe_route<<<1, kRouteThreads, 0, st>>>(ids, npairs, top_k, n_experts, pad, tile,
-                                             moe_max_rows(npairs, n_experts, pad), pos, row_tok, mt, ntm);
+    k_moe_route<<<1, kRouteThreads, 0, st>>>(ids, npairs, top_k, n_experts, pad, tile, pos, scratch, mt, ntm);
     return hipGetLastError();
 }
 

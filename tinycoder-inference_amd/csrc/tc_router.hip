@@ -158,37 +158,38 @@ __global__ __launch_bounds__(64) void k_router_logits(const float *__restrict__ 
     finish<TS, TE>(a, lane, s0, r0, S, rows, cols, X, W, out);
 }
 
-// Many tokens: a workgroup of 4 half-waves (2 x 2 blocks of 8 x 8) computes
+// Many tokens: a workgroup of 8 half-waves (4 x 2 blocks of 4 x 8) computes
 // 16 tokens x 16 rows from 128-column chunks in LDS, loaded one chunk ahead:
-// 64 FMAs per 16 LDS reads (at a row stride that puts the two row blocks that
-// a wave reads at once on different banks). cols % kChunk == 0.
+// 32 FMAs per 12 LDS reads (at a row stride that puts the two row blocks that
+// a wave reads at once on different banks). cols % kChunk == 0. (8 x 8 blocks,
+// half the waves: 25.0 against 20.5 us at 1024 tokens x 128 experts x 2048.)
 constexpr uint32_t kTile = 16, kChunk = 128;
 typedef float f4 __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(128) void k_router_logits_tiled(const float *__restrict__ W, const float *__restrict__ X,
+__global__ __launch_bounds__(256) void k_router_logits_tiled(const float *__restrict__ W, const float *__restrict__ X,
                                                              uint32_t S, uint32_t rows, uint32_t cols,
                                                              float *__restrict__ out) {
     __shared__ __align__(16) float lds[2][2 * kTile][kChunk + 4];  // tokens, then rows
     const uint32_t tid = threadIdx.x, lane = tid & 31, hw = tid >> 5;
     const uint32_t r0 = blockIdx.x * kTile, s0 = blockIdx.y * kTile;
-    const uint32_t hs = 8 * (hw >> 1), hr = 8 * (hw & 1);
-    constexpr int NL = 2 * kTile * kChunk / 4 / 128;  // float4 loads per thread and chunk
+    const uint32_t hs = 4 * (hw >> 1), hr = 8 * (hw & 1);
+    constexpr int NL = 2 * kTile * kChunk / 4 / 256;  // float4 loads per thread and chunk
     f4 v[NL];
-    // load k of this thread: columns 4 lane .. + 3 of row 4 k + hw of the chunk
+    // load k of this thread: columns 4 lane .. + 3 of row 8 k + hw of the chunk
     auto load = [&](uint32_t c) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < NL; ++k) {
-            const uint32_t q = 4 * k + hw;
+            const uint32_t q = 8 * k + hw;
             const float *p = q < kTile ? X + size_t(min(s0 + q, S - 1)) * cols : W + size_t(min(r0 + q - kTile, rows - 1)) * cols;
             v[k] = *reinterpret_cast<const f4 *>(p + c + 4 * lane);
         }
     };
     auto store = [&](uint32_t b) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < NL; ++k) *reinterpret_cast<f4 *>(&lds[b][4 * k + hw][4 * lane]) = v[k];
+        for (int k = 0; k < NL; ++k) *reinterpret_cast<f4 *>(&lds[b][8 * k + hw][4 * lane]) = v[k];
     };
-    float a[64];
+    float a[32];
 #pragma unroll
-    for (int o = 0; o < 64; ++o) a[o] = 0.0f;
+    for (int o = 0; o < 32; ++o) a[o] = 0.0f;
     const uint32_t nchunk = cols / kChunk;
     load(0);
     store(0);
@@ -198,19 +199,19 @@ __global__ __launch_bounds__(128) void k_router_logits_tiled(const float *__rest
         const uint32_t b = c & 1;
 #pragma unroll
         for (int i = 0; i < int(kChunk / 32); ++i) {
-            float xv[8], wv[8];
+            float xv[4], wv[8];
 #pragma unroll
-            for (int t = 0; t < 8; ++t) xv[t] = lds[b][hs + t][32 * i + lane];
+            for (int t = 0; t < 4; ++t) xv[t] = lds[b][hs + t][32 * i + lane];
 #pragma unroll
             for (int e = 0; e < 8; ++e) wv[e] = lds[b][kTile + hr + e][32 * i + lane];
 #pragma unroll
-            for (int t = 0; t < 8; ++t)
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) a[t * 8 + e] = fmaf(xv[t], wv[e], a[t * 8 + e]);
         }
         if (c + 1 < nchunk) store(b ^ 1);
     }
-    finish<8, 8>(a, lane, s0 + hs, r0 + hr, S, rows, cols, X, W, out);
+    finish<4, 8>(a, lane, s0 + hs, r0 + hr, S, rows, cols, X, W, out);
 }
 
 // ---- selection --------------------------------------------------------------
@@ -392,14 +393,14 @@ hipError_t launch_router_logits(const float *W, const float *X, uint32_t S, uint
     if (S == 0 || rows == 0 || cols == 0 || S > 65535) return hipErrorInvalidValue;
     // The largest block that still gives 512 half-waves or more (128 experts x
     // 2048 against one token x 8 rows per workgroup: the launch takes 3.1 us
-    // instead of 21 at 1 token, 25 instead of 182 at 1024); the tiled kernel
+    // instead of 21 at 1 token, 20.5 instead of 182 at 1024); the tiled kernel
     // needs 16-byte aligned rows of whole chunks.
     const uint64_t outs = uint64_t(S) * rows;
     const bool vec4 = cols % kChunk == 0 && (reinterpret_cast<uintptr_t>(W) & 15) == 0 &&
                       (reinterpret_cast<uintptr_t>(X) & 15) == 0;
     auto grid = [&](uint32_t ts, uint32_t te) { return dim3{(rows + 2 * te - 1) / (2 * te), (S + ts - 1) / ts, 1u}; };
     if (outs >= 512 * 64 && vec4)
-        k_router_logits_tiled<<<dim3{(rows + kTile - 1) / kTile, (S + kTile - 1) / kTile, 1u}, 128, 0, st>>>(W, X, S, rows,
+        k_router_logits_tiled<<<dim3{(rows + kTile - 1) / kTile, (S + kTile - 1) / kTile, 1u}, 256, 0, st>>>(W, X, S, rows,
                                                                                                           cols, out);
     else if (outs >= 512 * 16)
         k_router_logits<4, 4, 4><<<grid(4, 4), 64, 0, st>>>(W, X, S, rows, cols, out);

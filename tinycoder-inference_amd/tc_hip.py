@@ -112,8 +112,14 @@ class Library:
 
     # -- helpers ---------------------------------------------------------------
     def _stream(self):
+        # The current device's current stream as a handle: reading it without
+        # building a torch.cuda.Stream object takes 0.4 instead of 2.9 us, a
+        # quarter of a small call's host time (10.1 -> 7.6 us for tc_gemv).
         import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is None:
+            return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return ctypes.c_void_p(raw(torch.cuda.current_device()))
 
     def _check(self, rc):
         if rc != TC_OK:

@@ -154,6 +154,29 @@ def test_gemm_fp32_activations_nonfinite(tc, dev, oracle, qt):
     assert np.array_equal(got[keep], clean[keep])
 
 
+# Q8_0 rows of an even number of 32-blocks, read in place: widths below and
+# above 256, 2, 4 and 6 blocks left, every tile geometry (64 and 128 tokens, 256
+# rows from 257 tokens), split tiles. A NaN or infinite scale in the next row's
+# first blocks, which the last superblock's loads bring in, changes nothing.
+@pytest.mark.parametrize("M,N,K", [(1, 1, 64), (9, 40, 192), (33, 130, 320), (64, 77, 448), (65, 257, 1088),
+                                   (128, 300, 2880), (129, 129, 576), (257, 500, 2880), (300, 1030, 832)])
+def test_gemm_q80_ragged_in_place(tc, dev, oracle, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    w = random_blocks(Q8_0, rng, N, K)
+    x = gaussian(rng, (M, K))
+    ref = oracle_matmul_par(oracle, Q8_0, w, x, N, K)
+    got = tc.gemm(Q8_0, to_dev(w, dev), to_dev(x, dev), N, K).cpu().numpy()
+    ok, worst = close(got, ref)
+    assert ok, f"M={M} N={N} K={K}: worst err/bound {worst:.3g}"
+    if N > 2:
+        bad = w.reshape(N, K // 32, 34).copy()
+        bad[1, 0, :2] = np.frombuffer(np.float16(np.nan).tobytes(), np.uint8)
+        bad[N - 1, 1, :2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+        got2 = tc.gemm(Q8_0, to_dev(bad.ravel(), dev), to_dev(x, dev), N, K).cpu().numpy()
+        keep = [n for n in range(N) if n not in (1, N - 1)]
+        assert np.array_equal(got2[:, keep], got[:, keep])
+
+
 @pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ2_XS, IQ4_XS, IQ4_NL, Q5_0])
 def test_gemm_exact_batched_types(tc, dev, oracle, qt):
     rng = np.random.default_rng(5 + qt)

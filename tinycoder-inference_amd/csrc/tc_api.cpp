@@ -270,13 +270,14 @@ size_t gemm_mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int
 // (partials in ws when the split needs them). No allocation.
 int gemm_mfma_into(int type, const void *w, const float *x, float *out, uint32_t S, uint32_t rows, uint32_t cols,
                    int num_cu, void *act, void *ws, hipStream_t st) {
-    const tc::ActLayout L = tc::act_layout(type, S, cols);
+    const uint32_t ac = (cols + 255) / 256 * 256;  // the activations' width (ragged Q8_0: zeros past cols)
+    const tc::ActLayout L = tc::act_layout(type, S, ac);
     // the quantizer also zeroes the prefill GEMM's arrival counters (the
     // head of ws)
-    const uint32_t nctr = ws ? tc::prefill_counter_words(type, S, rows, cols, num_cu) : 0;
-    hipError_t e = tc::launch_quant_act(type, x, S, cols, L, act, st, true, static_cast<uint32_t *>(ws), nctr);
+    const uint32_t nctr = ws ? tc::prefill_counter_words(type, S, rows, ac, num_cu) : 0;
+    hipError_t e = tc::launch_quant_act(type, x, S, ac, L, act, st, true, static_cast<uint32_t *>(ws), nctr, cols);
     if (e != hipSuccess) return hip_fail(e, "activation quantizer");
-    e = tc::launch_prefill(type, w, act_view(act, L, 0, type, cols), out, S, rows, cols, num_cu, ws, st);
+    e = tc::launch_prefill(type, w, act_view(act, L, 0, type, ac), out, S, rows, cols, num_cu, ws, st);
     if (e != hipSuccess) return hip_fail(e, "int8 MFMA GEMM");
     return TC_OK;
 }
@@ -295,6 +296,15 @@ int fail_code(int code, const char *msg) { return fail(code, "%s", msg); }
 }  // namespace tc
 
 namespace {
+
+// The library's buffers, grown for one MFMA GEMM call.
+int gemm_scratch(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols) {
+    size_t act_bytes = 0;
+    const size_t ws = tc::gemm_mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
+    if (!ensure(dev->act, dev->act_bytes, act_bytes)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", act_bytes);
+    if (!ensure(dev->aux, dev->aux_bytes, ws)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", ws);
+    return TC_OK;
+}
 
 // The exact batched path (the reference's launchQGemm,
 // GpuGemvIQInt8.hpp:771-847): the decode kernel over token groups.
@@ -470,6 +480,15 @@ int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_le
     if (ragged_q80(type, cols)) {
         if (uint64_t(seq_len) * cols >= (uint64_t(1) << 30))
             return fail(TC_E_UNSUPPORTED, "activations of 4 GiB or more");
+        const uint32_t cp = (cols + 255) / 256 * 256;
+        if (cols % 64 == 0) {
+            // an even number of 32-blocks keeps the rows 4-byte aligned, which
+            // the MFMA kernel's loads need: no padded copies (4001x2880 at
+            // 333 tokens: 54.4 -> 38.7 us)
+            if ((rc = tc::gemm_mfma_check(type, seq_len, rows, cp))) return rc;
+            if ((rc = gemm_scratch(dev, type, seq_len, rows, cp))) return rc;
+            return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
+        }
         Padded p;
         if ((rc = pad_q80(dev, w, nullptr, rows, x, seq_len, cols, &p, st))) return rc;
         w = p.w[0];
@@ -495,11 +514,8 @@ int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_le
         return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
     }
     if ((rc = tc::gemm_mfma_check(type, seq_len, rows, cols))) return rc;
-    size_t act_bytes = 0;
-    const size_t ws = tc::gemm_mfma_scratch(type, seq_len, rows, cols, dev->num_cu, &act_bytes);
-    if (!ensure(dev->act, dev->act_bytes, act_bytes)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", act_bytes);
-    if (ws && !ensure(dev->aux, dev->aux_bytes, ws)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", ws);
-    return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, ws ? dev->aux : nullptr, st);
+    if ((rc = gemm_scratch(dev, type, seq_len, rows, cols))) return rc;
+    return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
 }
 
 int tc_gemm_preferred(uint32_t type, uint32_t, uint32_t) { return type_ok(int(type)) ? 1 : 0; }

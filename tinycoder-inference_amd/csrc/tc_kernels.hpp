@@ -12,10 +12,12 @@ namespace tc {
 // With block_major the blocks are stored block-major (block j of token t at
 // j * S + t), the layout launch_prefill reads.
 // The launch also zeroes zero[0 .. nzero) (the prefill GEMM's arrival
-// counters, which must be zero when the GEMM that follows starts).
+// counters, which must be zero when the GEMM that follows starts). xcols (Q8_0,
+// a multiple of 32 up to cols; 0: cols): the width of x, quantized as if
+// zeros followed to cols.
 hipError_t launch_quant_act(int wtype, const float *x, uint32_t S, uint32_t cols, const ActLayout &L,
                             void *buf, hipStream_t st, bool block_major = false, uint32_t *zero = nullptr,
-                            uint32_t nzero = 0);
+                            uint32_t nzero = 0, uint32_t xcols = 0);
 
 // Q8_K block-major quantization of x[T][cols] into the T * top_k rows of L: row
 // pos[t * top_k + r] is token t (negative: none). No bsums.
@@ -26,8 +28,8 @@ hipError_t launch_quant_act_scatter(const float *x, const int32_t *pos, uint32_t
 // Weight encoder: x[nunits][256] fp32 -> nunits units of `type`.
 hipError_t launch_encode(int type, const float *x, void *out, uint32_t nunits, hipStream_t st);
 
-// rows x src_row_bytes -> rows x dst_row_bytes (a multiple of 4), each row
-// copied and zero-filled past src_row_bytes.
+// rows x src_row_bytes -> rows x dst_row_bytes (a multiple of 16, dst 16-byte
+// and src 4-byte aligned), each row copied and zero-filled past src_row_bytes.
 hipError_t launch_pad_rows(const void *src, uint32_t src_row_bytes, void *dst, uint32_t dst_row_bytes, uint32_t rows,
                            hipStream_t st);
 
@@ -84,7 +86,8 @@ uint32_t gemv_max_tokens(int type, uint32_t cols);
 // Stream-K over one workgroup per CU. Q4_K, Q5_K and Q8_0 need the
 // activations' scale data (act.dg); every type prefill_workspace_bytes() of scratch
 // whose first prefill_counter_words() 32-bit words are zero when the launch
-// starts (every launch leaves them zero again).
+// starts (every launch leaves them zero again). Q8_0 also takes K % 64 == 0,
+// with the activations (and the sizes asked for) of K rounded up to 256.
 bool prefill_type(int type);
 uint32_t prefill_counter_words(int type, uint32_t M, uint32_t N, uint32_t K, int num_cu);
 size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int num_cu);

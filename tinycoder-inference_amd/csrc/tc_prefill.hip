@@ -107,6 +107,16 @@ template <>
 struct PfType<kQ8W> {
     static constexpr uint32_t PR = 256, TSPLIT = 1, UB = 272, XB = 64;
 };
+// Both for rows of an even number of 32-blocks that is no multiple of 8: rows
+// start 4-byte aligned, and the last superblock's missing blocks (the next
+// row's first ones in LDS) get scale 0 against activations that are 0.
+constexpr int kQ8R = 109, kQ8RW = 110;
+template <>
+struct PfType<kQ8R> : PfType<kQ8_0> {};
+template <>
+struct PfType<kQ8RW> : PfType<kQ8W> {};
+__host__ __device__ constexpr bool pf_q8(int type) { return type == kQ8_0 || (type >= kQ8W && type <= kQ8RW); }
+__host__ __device__ constexpr bool pf_q8_ragged(int type) { return type == kQ8R || type == kQ8RW; }
 // Q6_K: the 210-byte unit (2-byte aligned) in the 224-byte window from its
 // 4-byte-aligned start (14 chunks, loaded as 15 at a 240-byte row stride:
 // conflict-free 16-byte reads); at most 64 tokens per tile (256 such rows
@@ -168,7 +178,7 @@ __host__ __device__ constexpr uint32_t pf_grid_bytes(int type) {
 // next superblock's weights are loaded only after a barrier that follows
 // those reads (the activations stay double-buffered).
 template <int TYPE, int NT>
-constexpr bool pf_shared_w() { return ((TYPE == kQ5_K || TYPE == kQ6_K) && NT == 4) || TYPE == kQ8W; }
+constexpr bool pf_shared_w() { return ((TYPE == kQ5_K || TYPE == kQ6_K) && NT == 4) || TYPE == kQ8W || TYPE == kQ8RW; }
 template <int TYPE, int NT>
 struct PLds {
     using T = PfType<TYPE>;
@@ -179,7 +189,7 @@ struct PLds {
     static constexpr uint32_t QS = 0;
     static constexpr uint32_t XS = TT * 256;
     static constexpr uint32_t D8 = XS + TT * T::XB;
-    static constexpr uint32_t W = D8 + (TYPE != kQ8_0 && TYPE != kQ8W ? (TT < 64 ? 64 : TT) * 4 : 0);
+    static constexpr uint32_t W = D8 + (!pf_q8(TYPE) ? (TT < 64 ? 64 : TT) * 4 : 0);
     static constexpr uint32_t TAIL = W + (SW ? 0 : T::PR * T::UB);
     static constexpr uint32_t bytes = TAIL + (TYPE == kIQ3_XXS ? T::PR * 4 : 0);
     static constexpr uint32_t WS = BUF0 + 2 * bytes;  // the shared weight region (SW)
@@ -731,7 +741,9 @@ struct Q8Frag {
     v4i bw[8], bp[8];
 };
 
-__device__ __forceinline__ void q8_convert(const unsigned char *row, uint32_t g, Q8Frag &f) {
+// RAGGED: only the first nv blocks exist (their scales alone are taken).
+template <bool RAGGED>
+__device__ __forceinline__ void q8_convert(const unsigned char *row, uint32_t g, uint32_t nv, Q8Frag &f) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         // the 16 values start at byte 34k + 2 + 16g: in the 16-byte chunks
@@ -750,7 +762,7 @@ __device__ __forceinline__ void q8_convert(const unsigned char *row, uint32_t g,
             f.bw[k][i] = sh % 4 == 0 ? int(v[sh / 4 + i])
                                      : int(__builtin_amdgcn_alignbyte(v[sh / 4 + i + 1], v[sh / 4 + i], sh % 4));
         const uint32_t dword = lds1(row + ((34 * k) & ~3u));
-        const uint32_t dbits = (k & 1) ? dword >> 16 : dword & 0xFFFFu;
+        const uint32_t dbits = RAGGED && uint32_t(k) >= nv ? 0u : (k & 1) ? dword >> 16 : dword & 0xFFFFu;
         const float d = h2f(dbits);
         const uint32_t hb = __builtin_bit_cast(uint32_t, d) & 0xFFFF0000u;
         const uint32_t lb = __builtin_bit_cast(uint32_t, d - __builtin_bit_cast(float, hb));
@@ -975,7 +987,7 @@ __device__ __forceinline__ void stage(const PfArgs &a, const uint8_t *W, uint32_
         lds_load16(base + L::QS + 1024 * k, rq, (tb + t) * 256 + 16 * ((ln & 15) ^ (t & 15)));
     });
     const v4i rx = rs4(a.xs, a.M * a.nblk * T::XB);
-    if constexpr (TYPE != kQ8_0 && TYPE != kQ8W) {
+    if constexpr (!pf_q8(TYPE)) {
         if constexpr (T::XB != 0)
             each_inst<TT / 32>(w, [&](uint32_t k) {
                 lds_load16(base + L::XS + 1024 * k, rx, (tb + 32 * k) * T::XB + 16 * ln);
@@ -1241,7 +1253,7 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 }
             } else {
                 Q8Frag f;
-                q8_convert(wb + rl * T::UB, g, f);
+                q8_convert<pf_q8_ragged(TYPE)>(wb + rl * T::UB, g, a.nb32 - 8 * b, f);
                 if constexpr (L::SW) {
                     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): every raw read done
                     __syncthreads();
@@ -1514,9 +1526,12 @@ size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int
 
 hipError_t launch_prefill(int type, const void *W, const ActView &act, float *out, uint32_t M, uint32_t N,
                           uint32_t K, int num_cu, void *workspace, hipStream_t st) {
-    if (!prefill_type(type) || M == 0 || N == 0 || K == 0 || K % 256 || workspace == nullptr ||
+    const bool ragged = type == kQ8_0 && K % 256 != 0;
+    if (!prefill_type(type) || M == 0 || N == 0 || K == 0 || K % (ragged ? 64 : 256) || workspace == nullptr ||
         ((type == kQ4_K || type == kQ5_K || type == kQ8_0) && act.dg == nullptr))
         return hipErrorInvalidValue;
+    const uint32_t nb32 = K / 32;
+    K = (K + 255) / 256 * 256;  // (ragged Q8_0: the activations' width)
     if (uint64_t(M) * K >= (uint64_t(1) << 32) || uint64_t(N) * (K / 256) * unit_bytes(type) >= (uint64_t(1) << 32))
         return hipErrorInvalidValue;
     const PfGeom g = pf_geom(type, M, N, K, num_cu);
@@ -1532,12 +1547,17 @@ hipError_t launch_prefill(int type, const void *W, const ActView &act, float *ou
     a.N = N;
     a.K = K;
     a.nblk = K / 256;
-    a.row_bytes = a.nblk * unit_bytes(type);
+    a.nb32 = nb32;
+    a.row_bytes = type == kQ8_0 ? nb32 * 34 : a.nblk * unit_bytes(type);
     a.ntm = g.ntm;
     a.ntn = g.ntn;
     a.ntiles = g.ntiles;
     a.G = g.G;
     a.fused = g.fused ? 1u : 0u;
+    if (ragged) {
+        if (g.wide) return pf_launch<kQ8RW, 4>(a, st);
+        return g.nt == 2 ? pf_launch<kQ8R, 2>(a, st) : pf_launch<kQ8R, 4>(a, st);
+    }
     if (type == kQ8_0) {
         if (g.wide) return pf_launch<kQ8W, 4>(a, st);
         return g.nt == 2 ? pf_launch<kQ8_0, 2>(a, st) : pf_launch<kQ8_0, 4>(a, st);

@@ -41,6 +41,7 @@ struct PfArgs {
     // tiles of W2 / out2 follow those of W / out in one launch.
     const uint8_t *W2;
     float *out2;
+    uint32_t nb32;  // 32-blocks of a row (the last superblock of ragged Q8_0 rows has fewer than 8)
 };
 
 // A tile's token rows [m0, mend), weight matrix and output.

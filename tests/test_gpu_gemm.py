@@ -177,6 +177,39 @@ def test_gemm_q80_ragged_in_place(tc, dev, oracle, M, N, K):
         assert np.array_equal(got2[:, keep], got[:, keep])
 
 
+@pytest.mark.parametrize("S,N,K", [(8, 40, 18944), (5, 33, 18944), (4, 5000, 9216)])
+@pytest.mark.parametrize("qt", ALL)
+def test_few_tokens_on_the_matrix_cores(tc, dev, oracle, qt, S, N, K):
+    """tc_gemv (and tc_gemm) at 8 tokens or less where the decode kernel would
+    need several launches: the oracle's results, and under stream capture the
+    decode kernel's, on every replay."""
+    import torch
+    rng = np.random.default_rng(S + N + K + qt)
+    w = enc_weights(oracle, qt, rng, N, K) if N < 100 else random_blocks(qt, rng, N, K)
+    x = gaussian(rng, (S, K))
+    wd, xd = to_dev(w, dev), to_dev(x, dev)
+    got = tc.gemv(qt, wd, xd, N, K).cpu().numpy()
+    if N < 100:
+        ref = oracle_matmul_par(oracle, qt, w, x, N, K)
+        ok, worst = close(got, ref)
+        assert ok, f"{NAMES[qt]} S={S} N={N} K={K}: worst err/bound {worst:.3g}"
+        assert np.array_equal(tc.gemm(qt, wd, xd, N, K).cpu().numpy(), got) or qt in MFMA_TYPES
+    out = torch.empty((S, N), device=dev)
+    for i in range(S):  # the warm-up: the decode kernel's own launches
+        tc.gemv(qt, wd, xd[i:i + 1].contiguous(), N, K)
+    tc._check(tc.lib.tc_gemv_reserve(K, 8))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tc.gemv(qt, wd, xd, N, K, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        d = np.abs(out.cpu().numpy() - got)
+        assert d.max() <= 1e-5 * np.abs(got).max(), f"{NAMES[qt]}: {d.max()}"
+
+
 @pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ2_XS, IQ4_XS, IQ4_NL, Q5_0])
 def test_gemm_exact_batched_types(tc, dev, oracle, qt):
     rng = np.random.default_rng(5 + qt)

@@ -98,7 +98,7 @@ bool g_q8_gemm_enabled = true;
 
 // Weight types that always run the int8 MFMA prefill GEMM (and the only ones
 // tc_gemm_noalloc takes). The others have the decode kernel over groups of 8
-// tokens behind the matrix-core kernel: see gemm_route_mfma.
+// tokens behind the matrix-core kernel: see route_mfma.
 bool mfma_gemm_type(int t) {
     return t == TC_Q4_K || t == TC_Q5_K || t == TC_Q6_K || t == TC_IQ3_XXS || t == TC_IQ3_S || t == TC_IQ2_S || t == TC_Q8_0;
 }
@@ -325,16 +325,39 @@ uint32_t gemm_f32_chunk(uint32_t cols) {
     return std::max(256u, uint32_t((size_t(96) << 20) / (size_t(cols) * 6)) / 128 * 128);
 }
 
-// Whether a product of one of the types that also have the batched path goes
-// to the matrix cores; its scratch is in place then. Up to 8 tokens the
-// batched path is one launch that reads the weights once (Q3_K 18944x3584, 8
-// tokens: 29 us against 45). It also keeps the calls that need more than 32-bit
-// offsets or than the memory left, and those under graph capture, which it
-// serves from less scratch or none (the MFMA path's could not grow there, and
-// its address would be held by the graph).
-bool gemm_route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
+// Whether up to 8 tokens go to the matrix cores rather than to the decode
+// kernel, which takes smax tokens per launch (its LDS holds their activations)
+// and reads the weights once per launch: from 3 launches on (small matrices of
+// the fp32-activation types from 5), and from 2 where that measured faster (us,
+// decode against MFMA: Q6_K 3584x18944 3 tokens 51 / 33, 8 tokens 137 / 33,
+// 256x18944 33 / 21 and 87 / 21; Q4_K 3584x18944 4 tokens 26 / 26, 8 tokens 45
+// / 26; Q5_K 3 tokens 28 / 32, 5000x9216 5 tokens 23 / 26; IQ4_NL 256x18944 3
+// tokens 21 / 28, 5 tokens 35 / 28; at 64 MB two decode launches' streams take
+// as long as the MFMA kernel's one). The fp32-activation types also where their
+// 512-thread launch no longer fits (18944x3584: IQ4_NL 4 tokens 49 / 37, 5
+// tokens 108 / 38; Q5_0 46 / 41; IQ2_XS 5 tokens 44 / 41).
+bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols) {
+    const uint32_t smax = tc::gemv_max_tokens(type, cols);
+    if (smax == 0 || (type == TC_Q8_0 && !g_q8_gemm_enabled)) return false;
+    const uint32_t launches = (S + smax - 1) / smax;
+    const uint64_t bytes = uint64_t(rows) * tc_row_bytes(type, cols);
+    if (launches >= (tc::prefill_f32_type(type) && bytes < (16u << 20) ? 5u : 3u)) return true;
+    if (bytes < (16u << 20) || bytes > (64u << 20)) return false;
+    if (launches == 2 && S >= (smax == 1 ? 2u : type == TC_Q5_K ? 6u : 4u)) return true;
+    return tc::prefill_f32_type(type) && S >= (type == TC_IQ2_XS ? 5u : 4u);
+}
+
+// Whether a call that the decode kernel could serve goes to the matrix cores;
+// its scratch is in place then. The decode kernel keeps calls of 8 tokens or
+// less but for the above, those that need more than 32-bit offsets or than the
+// memory left, and those under graph capture, which it serves from less
+// scratch or none (the MFMA path's could not grow there, and its address would
+// be held by the graph).
+bool route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
     const bool f32 = tc::prefill_f32_type(type);
-    if (S <= 8 || !(f32 || tc::prefill_type(type)) || !tc::gemm_mfma_addressable(type, S, rows, cols)) return false;
+    if ((S <= 8 && !few_tokens_mfma(type, S, rows, cols)) || !(f32 || tc::prefill_type(type)) ||
+        !tc::gemm_mfma_addressable(type, S, rows, cols))
+        return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (st != nullptr && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone))
         return false;
@@ -350,6 +373,20 @@ bool gemm_route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t 
     if (ensure(dev->act, dev->act_bytes, act_bytes) && ensure(dev->aux, dev->aux_bytes, ws)) return true;
     (void)hipGetLastError();  // the failed allocation's
     return false;
+}
+
+// The matrix-core product of a call that route_mfma took.
+int run_mfma(Device *dev, int type, const void *w, const float *x, float *out, uint32_t S, uint32_t rows, uint32_t cols,
+             hipStream_t st) {
+    if (!tc::prefill_f32_type(type))
+        return tc::gemm_mfma_into(type, w, x, out, S, rows, cols, dev->num_cu, dev->act, dev->aux, st);
+    const uint32_t chunk = gemm_f32_chunk(cols);
+    for (uint32_t s0 = 0; s0 < S; s0 += chunk) {
+        const hipError_t e = tc::launch_prefill_f32(type, w, x + size_t(s0) * cols, out + size_t(s0) * rows,
+                                                    std::min(chunk, S - s0), rows, cols, dev->num_cu, dev->act, dev->aux, st);
+        if (e != hipSuccess) return hip_fail(e, "bf16 MFMA GEMM");
+    }
+    return TC_OK;
 }
 
 }  // namespace
@@ -385,6 +422,8 @@ int tc_gemv(int type, const void *w, const float *x, float *out, uint32_t seq_le
         if ((rc = pad_q80(dev, w, nullptr, rows, x, seq_len, cols, &p, st))) return rc;
         return run_gemv(dev, type, p.w[0], nullptr, p.x, nullptr, out, nullptr, 0, nullptr, seq_len, rows, p.cols, st);
     }
+    if (seq_len > 1 && route_mfma(dev, type, seq_len, rows, cols, st))
+        return run_mfma(dev, type, w, x, out, seq_len, rows, cols, st);
     return run_gemv(dev, type, w, nullptr, x, nullptr, out, nullptr, 0, nullptr, seq_len, rows, cols, st);
 }
 
@@ -499,19 +538,9 @@ int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_le
         // Q2_K / Q3_K / IQ4_XS and the fp32-activation IQ2_XS / IQ4_NL / Q5_0
         if (tc::gemv_max_tokens(type, cols) == 0)
             return fail(TC_E_UNSUPPORTED, "cols=%u too wide for the decode kernel", cols);
-        if (!gemm_route_mfma(dev, type, seq_len, rows, cols, st))
+        if (!route_mfma(dev, type, seq_len, rows, cols, st))
             return gemm_batched(dev, type, w, x, out, seq_len, rows, cols, st);
-        if (tc::prefill_f32_type(type)) {
-            const uint32_t chunk = gemm_f32_chunk(cols);
-            for (uint32_t s0 = 0; s0 < seq_len; s0 += chunk) {
-                const hipError_t e =
-                    tc::launch_prefill_f32(type, w, x + size_t(s0) * cols, out + size_t(s0) * rows,
-                                           std::min(chunk, seq_len - s0), rows, cols, dev->num_cu, dev->act, dev->aux, st);
-                if (e != hipSuccess) return hip_fail(e, "bf16 MFMA GEMM");
-            }
-            return TC_OK;
-        }
-        return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
+        return run_mfma(dev, type, w, x, out, seq_len, rows, cols, st);
     }
     if ((rc = tc::gemm_mfma_check(type, seq_len, rows, cols))) return rc;
     if ((rc = gemm_scratch(dev, type, seq_len, rows, cols))) return rc;

@@ -33,9 +33,9 @@
 //    signs applied in registers.
 //  * Q2_K, Q3_K, IQ4_XS: as Q4_K (256 rows); conversions at each type below.
 //    18944x3584 against the decode kernel over groups of 8 tokens, which
-//    reads and decodes the weights once per group: Q3_K M = 512 1661 -> 75
-//    us (934 TOPS), M = 2048 6671 -> 253 us (1098 TOPS); Q2_K 2065 -> 91 and
-//    8234 -> 311; IQ4_XS 1498 -> 117 and 5705 -> 406.
+//    reads and decodes the weights once per group: Q3_K M = 512 1661 -> 83
+//    us (837 TOPS), M = 2048 6671 -> 280 us (994 TOPS); Q2_K M = 2048 8254 ->
+//    337, IQ4_XS 5524 -> 427.
 //
 // Q4_K (reference dequantizeQ4_KBlock, GGMLDequantize.hpp:436-477): a weight
 // of sub-block s is w = d*sc_s*q - dmin*m_s with q in 0..15 and sc_s, m_s in
@@ -177,6 +177,13 @@ __host__ __device__ constexpr uint32_t pf_grid_bytes(int type) {
 // buffers): each wave reads its rows' raw bytes into registers first, and the
 // next superblock's weights are loaded only after a barrier that follows
 // those reads (the activations stay double-buffered).
+// Q2_K, Q3_K and IQ4_XS hold the sum of at most pf_chain superblocks in the
+// accumulators, which then go into fp32 sums in memory, their rounding staying
+// behind in the accumulators (one fp32 chain over all of K was further from
+// the 64-bit results than the decode kernel's tree: Q3_K 3584x18944 M = 2048
+// 1.28e-7 against 0.79e-7, now 0.78e-7; 299 us instead of 270).
+__host__ __device__ constexpr uint32_t pf_chain(uint32_t nblk) { return nblk <= 48 ? 8 : 12; }
+__host__ __device__ constexpr bool pf_short_chain(int type) { return type == kQ2_K || type == kQ3_K || type == kIQ4_XS; }
 template <int TYPE, int NT>
 constexpr bool pf_shared_w() { return ((TYPE == kQ5_K || TYPE == kQ6_K) && NT == 4) || TYPE == kQ8W || TYPE == kQ8RW; }
 template <int TYPE, int NT>
@@ -1110,6 +1117,26 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 stage<TYPE, NT>(a, nt_.W, nt_.m0, nt_.n0, 0, buf(ph + 1), w, wbuf(ph + 1));
             }
         };
+        // Short chains: the accumulators into the thread's sums (behind the
+        // partial tiles, value r of token block t at (16 t + r) * 512 + the
+        // thread), or the sums back into them.
+        uint32_t held = 0;     // superblocks in acc
+        bool flushed = false;  // earlier ones are in the sums
+        auto spill = [&](bool back) __attribute__((always_inline)) {
+            float *const fl = a.ws + size_t(a.G) * 2 * (TT * PR) + size_t(v) * (TT * PR) + (64 * w + lane_now());
+#pragma unroll
+            for (int t = 0; t < NB; ++t) {
+                float p[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) p[r] = flushed ? fl[(16 * t + r) * 512] : 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float s = p[r] + acc[t][r];
+                    acc[t][r] = back ? s : acc[t][r] - (s - p[r]);
+                    if (!back) fl[(16 * t + r) * 512] = s;
+                }
+            }
+        };
         // Per superblock: its loads are waited for, the next superblock's
         // issued into the other LDS buffer, this lane's weights converted,
         // then the MFMAs.
@@ -1268,7 +1295,16 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
             __builtin_amdgcn_sched_barrier(0);
             ph ^= 1;
+            if constexpr (pf_short_chain(TYPE)) {
+                if (++held == pf_chain(a.nblk) && b + 1 < b1) {
+                    spill(false);
+                    held = 0;
+                    flushed = true;
+                }
+            }
         }
+        if constexpr (pf_short_chain(TYPE))
+            if (flushed) spill(true);
 
         // lane: row n0 + rl, tokens m0 + 32 (tg NB + t) + 8q + 4g + e
         const uint32_t n = n0 + rl;
@@ -1510,8 +1546,8 @@ bool prefill_type(int type) {
            type == kIQ2_S || type == kQ3_K || type == kQ2_K || type == kIQ4_XS;
 }
 
-// Workspace: the per-tile arrival counters (256-byte rounded), then the
-// partial tiles, two per workgroup.
+// Workspace: the per-tile arrival counters (256-byte rounded), the partial
+// tiles, two per workgroup, and the short-chain types' sums.
 namespace {
 size_t ctr_bytes(uint64_t ntiles) { return (ntiles * 4 + 255) & ~uint64_t(255); }
 }  // namespace
@@ -1521,7 +1557,8 @@ uint32_t prefill_counter_words(int type, uint32_t M, uint32_t N, uint32_t K, int
 size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int num_cu) {
     if (!prefill_type(type)) return 0;
     const PfGeom g = pf_geom(type, M, N, K, num_cu);
-    return ctr_bytes(g.ntiles) + size_t(g.G) * 2 * g.tt * g.pr * 4;
+    const size_t part = size_t(g.G) * 2 * g.tt * g.pr * 4;
+    return ctr_bytes(g.ntiles) + part + (pf_short_chain(type) && K / 256 > pf_chain(K / 256) ? part / 2 : 0);  // + the sums
 }
 
 hipError_t launch_prefill(int type, const void *W, const ActView &act, float *out, uint32_t M, uint32_t N,

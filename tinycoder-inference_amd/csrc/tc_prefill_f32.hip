@@ -441,7 +441,7 @@ hipError_t f_launch(const PfArgs &a, hipStream_t st) {
     k_prefill_f32<TYPE, RB, TB, TG><<<dim3{a.G, 1u, 1u}, 64 * PW, L::total, st>>>(a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || !pf_splits(a.ntiles * a.nblk, a.G, a.nblk)) return e;
-    k_pf_fixup<TT, kRows, false, double><<<dim3{(a.G - 1) * kFixSlices(TT, kRows), 1u, 1u}, 256, 0, st>>>(a);
+    k_pf_fixup<TT, kRows, false><<<dim3{(a.G - 1) * kFixSlices(TT, kRows), 1u, 1u}, 256, 0, st>>>(a);
     return hipGetLastError();
 }
 template <int TYPE>

@@ -81,8 +81,11 @@ int tc_act_quantize(int type, const float *x, uint32_t seq_len, uint32_t cols, v
 int tc_gemv_q8(int type, const void *w, const void *act, float *out, uint32_t seq_len, uint32_t rows,
                uint32_t cols, void *stream);
 
-/* Pre-size the activation scratch so that later tc_gemv / tc_gemm calls of
- * at most this size allocate nothing (e.g. before a hipGraph capture).
+/* Pre-size the scratch so that later tc_gemv / tc_gemm calls of at most this
+ * size allocate nothing (e.g. before a hipGraph capture), for every type, up to
+ * 1048576 rows (but Q8_0 at cols % 256 != 0, whose padded copies of the
+ * weights go by rows). A buffer that a captured call uses is kept when a later,
+ * larger call grows the scratch, so its graph stays valid.
  * Replaces tinycoder::gpu::int8GemvReserve (include/Int8Gemm.hpp:82). */
 int tc_gemv_reserve(uint32_t cols, uint32_t seq_len);
 

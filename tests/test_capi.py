@@ -132,3 +132,117 @@ def test_cpp_interface_driver_without_gpu():
     for t in (12, 11, 14, 13, 23, 20, 8):
         assert d.drv_matMulVecBatch_SIMD(t, w.ctypes.data, x.ctypes.data, 1, 1, 256, out.ctypes.data, None) == 0
     assert out[0] == 7.0
+
+
+def _compile_and_run(tmp_path, source, *args):
+    """A host program over the library's internal headers and functions."""
+    import shutil
+    import subprocess
+    import tc_hip
+    import torch  # noqa: F401  (its HIP runtime's folder, for the library)
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no host C++ compiler")
+    src = tmp_path / "prog.cpp"
+    src.write_text(source)
+    exe = tmp_path / "prog"
+    so = tc_hip.load_library()._name
+    subprocess.run([gxx, "-std=c++17", "-I", os.path.join(ROOT, "tinycoder-inference_amd", "csrc"), str(src), *args,
+                    so, "-Wl,-rpath," + os.path.dirname(so), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+
+
+def test_reserved_scratch_covers_every_route(tmp_path):
+    """tc_gemv_reserve's sizes cover what any tc_gemv or tc_gemm call of at most
+    the reserved tokens and columns asks of the two buffers, over all types,
+    token counts around every tile width, narrow to wide inputs and rows up
+    to the documented bound (such a call must not replace a buffer whose address
+    a graph holds)."""
+    import tc_hip
+    types = ", ".join(str(t) for t in tc_hip.TYPES.values())
+    _compile_and_run(tmp_path, r"""
+#include <stdint.h>
+#include <stdio.h>
+namespace tc {
+size_t mfma_scratch(int, uint32_t, uint32_t, uint32_t, int, size_t *);
+size_t reserve_scratch(uint32_t, uint32_t, int, size_t *);
+uint32_t gemv_max_tokens(int, uint32_t);
+}
+int main() {
+    const uint32_t tokens[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 32, 33, 64, 65, 100, 128, 129, 256, 257, 333, 1000, 2048, 6000};
+    const uint32_t cols[] = {256, 2304, 4096, 8192, 14336, 18944, 28672};
+    const uint32_t rows[] = {1, 255, 256, 3584, 18944, 19712, 128256, 152064, 1u << 20};
+    const int types[] = {""" + types + r"""};
+    for (uint32_t rs : tokens)
+        for (uint32_t rc : cols) {
+            size_t ract = 0;
+            const size_t raux = tc::reserve_scratch(rs, rc, 256, &ract);
+            for (uint32_t s : tokens)
+                for (uint32_t c : cols)
+                    for (uint32_t n : rows)
+                        for (int t : types) {
+                            if (s > rs || c > rc || tc::gemv_max_tokens(t, c) == 0) continue;
+                            size_t act = 0;
+                            const size_t aux = tc::mfma_scratch(t, s, n, c, 256, &act);
+                            if (act <= ract && aux <= raux) continue;
+                            printf("reserved %u x %u: %zu, %zu; type %d, %u tokens, %u x %u: %zu, %zu\n", rs, rc, ract,
+                                   raux, t, s, n, c, act, aux);
+                            return 1;
+                        }
+        }
+    return 0;
+}
+""")
+
+
+def test_scratch_growth_rule(tmp_path):
+    """Buffers that a graph may use are kept when they grow, and the kept ones
+    stay smaller than the one in use; a failed growth leaves a buffer as it was
+    unless the call cannot do without it."""
+    _compile_and_run(tmp_path, r"""
+#include <set>
+#include "tc_scratch.hpp"
+struct Mem {
+    size_t *room;
+    std::set<void *> *live, *gone;
+    void *alloc(size_t n) {
+        if (n > *room) return nullptr;
+        void *p = new char;
+        live->insert(p);
+        return p;
+    }
+    void release(void *p) {
+        live->erase(p);
+        gone->insert(p);
+        *room = 1000;
+    }
+};
+#define CHECK(c) do { if (!(c)) return __LINE__ % 256; } while (0)
+int main() {
+    size_t room = 1 << 30;
+    std::set<void *> live, gone;
+    Mem m{&room, &live, &gone};
+    tc::Scratch s;
+    CHECK(tc::scratch_grow(s, 100, false, true, m) && s.bytes == 100 && !s.held);
+    void *p = s.p;
+    CHECK(tc::scratch_grow(s, 200, false, true, m) && s.bytes == 200 && gone.count(p));  // no graph: given back
+    p = s.p;
+    CHECK(tc::scratch_grow(s, 150, true, true, m) && s.p == p && s.held);  // recorded
+    CHECK(tc::scratch_grow(s, 210, false, true, m) && s.p != p && s.bytes == 400 && live.count(p) && !s.held);
+    p = s.p;
+    CHECK(tc::scratch_grow(s, 500, true, true, m) && live.count(p) && s.held);  // grown while recording
+    p = s.p;
+    room = 0;
+    CHECK(!tc::scratch_grow(s, 5000, false, true, m) && s.p == p && s.held);  // held: kept at any rate
+    room = 1200;
+    CHECK(tc::scratch_grow(s, 1100, false, true, m) && s.bytes == 1100 && live.count(p));  // twice does not fit
+    p = s.p;
+    room = 0;
+    CHECK(!tc::scratch_grow(s, 1500, false, false, m) && s.p == p && s.bytes == 1100);  // optional: left alone
+    CHECK(tc::scratch_grow(s, 900, false, false, m) && s.p == p);
+    CHECK(!tc::scratch_grow(s, 1500, false, true, m) && gone.count(p) && s.p == nullptr && s.bytes == 0);
+    CHECK(tc::scratch_grow(s, 1000, false, true, m) && s.bytes == 1000);
+    return 0;
+}
+""")

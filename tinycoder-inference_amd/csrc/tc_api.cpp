@@ -14,6 +14,7 @@
 
 #include "tc_kernels.hpp"
 #include "tc_qmatmul.h"
+#include "tc_scratch.hpp"
 
 namespace {
 
@@ -37,12 +38,9 @@ int hip_fail(hipError_t e, const char *what) {
 struct Device {
     bool ok = false;
     int id = 0, num_cu = 0;
-    void *act = nullptr;  // quantized activations
-    size_t act_bytes = 0;
-    void *aux = nullptr;  // kernel intermediates (MoE hidden, GEMM partials)
-    size_t aux_bytes = 0;
-    void *pad = nullptr;  // zero-padded copies of Q8_0 rows of a width not a multiple of 256
-    size_t pad_bytes = 0;
+    tc::Scratch act;  // quantized activations
+    tc::Scratch aux;  // kernel intermediates (MoE hidden, GEMM partials)
+    tc::Scratch pad;  // zero-padded copies of Q8_0 rows of a width not a multiple of 256
 };
 
 std::mutex g_mu;
@@ -67,21 +65,29 @@ Device *device() {
     return &d;
 }
 
-bool ensure(void *&p, size_t &cap, size_t need) {
-    if (cap >= need) return true;
-    if (p != nullptr) {
+struct DeviceMem {
+    void *alloc(size_t n) {
+        void *p = nullptr;
+        if (hipMalloc(&p, n) == hipSuccess) return p;
+        (void)hipGetLastError();  // the failed allocation's
+        return nullptr;
+    }
+    void release(void *p) {
         // The buffer may still be read by work queued earlier on any stream.
         (void)hipDeviceSynchronize();
         (void)hipFree(p);
     }
-    p = nullptr;
-    cap = 0;
-    if (hipMalloc(&p, need) != hipSuccess) {
-        p = nullptr;
-        return false;
-    }
-    cap = need;
-    return true;
+};
+
+// Whether calls on st are being recorded into a graph (the null stream cannot be).
+bool recording(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return st != nullptr && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone);
+}
+
+// s grown to `need` bytes for a call on st.
+bool ensure(tc::Scratch &s, size_t need, hipStream_t st) {
+    return need == 0 || tc::scratch_grow(s, need, recording(st), true, DeviceMem{});
 }
 
 // Bytes past a GEMM activation buffer that the MFMA kernel's tail loads may
@@ -130,12 +136,12 @@ int launch_jobs(Device *dev, int type, uint32_t S, tc::GemvJob *jobs, uint32_t n
     for (uint32_t i = 0; i < n; ++i)
         if (jobs[i].x && prequantize_wide(type, S, jobs[i].cols, wbytes)) need += tc::act_layout(type, S, jobs[i].cols).bytes;
     if (need) {
-        if (!ensure(dev->act, dev->act_bytes, need)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", need);
+        if (!ensure(dev->act, need, st)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", need);
         size_t off = 0;
         for (uint32_t i = 0; i < n; ++i) {
             if (!(jobs[i].x && prequantize_wide(type, S, jobs[i].cols, wbytes))) continue;
             const tc::ActLayout L = tc::act_layout(type, S, jobs[i].cols);
-            void *buf = static_cast<char *>(dev->act) + off;
+            void *buf = static_cast<char *>(dev->act.p) + off;
             hipError_t e = tc::launch_quant_act(type, jobs[i].x, S, jobs[i].cols, L, buf, st);
             if (e != hipSuccess) return hip_fail(e, "activation quantizer");
             jobs[i].act = act_view(buf, L, 0, type, jobs[i].cols);
@@ -215,8 +221,8 @@ int pad_q80(Device *dev, const void *w0, const void *w1, uint32_t rows, const fl
     const uint32_t rb = cols / 32 * 34, rbp = cp / 32 * 34;
     const size_t wbytes = (size_t(rows) * rbp + 255) & ~size_t(255);
     const size_t need = wbytes * (w1 ? 2 : 1) + size_t(S) * cp * 4;
-    if (!ensure(dev->pad, dev->pad_bytes, need)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", need);
-    char *b = static_cast<char *>(dev->pad);
+    if (!ensure(dev->pad, need, st)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", need);
+    char *b = static_cast<char *>(dev->pad.p);
     hipError_t e = tc::launch_pad_rows(w0, rb, b, rbp, rows, st);
     if (e == hipSuccess && w1) e = tc::launch_pad_rows(w1, rb, b + wbytes, rbp, rows, st);
     if (e == hipSuccess && x) e = tc::launch_pad_rows(x, cols * 4, b + wbytes * (w1 ? 2 : 1), cp * 4, S, st);
@@ -293,16 +299,44 @@ int gemm_entry_check(int type, const void *w, const float *x, const float *out, 
 }
 
 int fail_code(int code, const char *msg) { return fail(code, "%s", msg); }
+
+// Tokens per launch of the fp32-activation MFMA kernel: the bf16 pieces take 6
+// bytes per value, so long prompts go in chunks of about 96 MB of pieces
+// (2048 tokens at 8192 columns).
+constexpr size_t kF32ChunkBytes = size_t(96) << 20;
+constexpr uint32_t kF32ChunkMin = 256;
+uint32_t gemm_f32_chunk(uint32_t cols) {
+    return std::max(kF32ChunkMin, uint32_t(kF32ChunkBytes / (size_t(cols) * 6)) / 128 * 128);
+}
+
+size_t mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu, size_t *act_bytes) {
+    if (!prefill_f32_type(type)) return gemm_mfma_scratch(type, S, rows, cols, num_cu, act_bytes);
+    const uint32_t n = std::min(S, gemm_f32_chunk(cols));
+    *act_bytes = prefill_f32_act_bytes(n, cols);
+    size_t ws = prefill_f32_workspace_bytes(n, rows, cols, num_cu);
+    if (S % n) ws = std::max(ws, prefill_f32_workspace_bytes(S % n, rows, cols, num_cu));
+    return ws;
+}
+
+size_t reserve_scratch(uint32_t S, uint32_t cols, int num_cu, size_t *act_bytes) {
+    *act_bytes = 0;
+    if (S == 0 || cols == 0) return 0;
+    const uint32_t cp = (cols + 255) / 256 * 256;  // (ragged Q8_0's activations)
+    for (int t : {TC_Q8_0, TC_Q4_K}) *act_bytes = std::max(*act_bytes, act_layout(t, S, cp).bytes + kGemmActSlack);
+    const size_t most = std::max(kF32ChunkBytes, prefill_f32_act_bytes(kF32ChunkMin, cp));
+    *act_bytes = std::max(*act_bytes, std::min(prefill_f32_act_bytes(S, cp), most));
+    return prefill_workspace_bound(S, kReserveRows, num_cu);
+}
 }  // namespace tc
 
 namespace {
 
 // The library's buffers, grown for one MFMA GEMM call.
-int gemm_scratch(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols) {
+int gemm_scratch(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
     size_t act_bytes = 0;
     const size_t ws = tc::gemm_mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
-    if (!ensure(dev->act, dev->act_bytes, act_bytes)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", act_bytes);
-    if (!ensure(dev->aux, dev->aux_bytes, ws)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", ws);
+    if (!ensure(dev->act, act_bytes, st)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", act_bytes);
+    if (!ensure(dev->aux, ws, st)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", ws);
     return TC_OK;
 }
 
@@ -316,13 +350,6 @@ int gemm_batched(Device *dev, int type, const void *w, const float *x, float *ou
         if (rc) return rc;
     }
     return TC_OK;
-}
-
-// Tokens per launch of the fp32-activation MFMA kernel: the bf16 pieces take 6
-// bytes per value, so long prompts go in chunks of about 96 MB of pieces
-// (2048 tokens at 8192 columns).
-uint32_t gemm_f32_chunk(uint32_t cols) {
-    return std::max(256u, uint32_t((size_t(96) << 20) / (size_t(cols) * 6)) / 128 * 128);
 }
 
 // Whether up to 8 tokens go to the matrix cores rather than to the decode
@@ -360,32 +387,22 @@ bool route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols,
     if ((S <= 8 && !few_tokens_mfma(type, S, rows, cols)) || !(f32 || tc::prefill_type(type)) ||
         !tc::gemm_mfma_addressable(type, S, rows, cols))
         return false;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (st != nullptr && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone))
-        return false;
-    size_t act_bytes = 0, ws = 0;
-    if (f32) {
-        const uint32_t n = std::min(S, gemm_f32_chunk(cols));
-        act_bytes = tc::prefill_f32_act_bytes(n, cols);
-        ws = tc::prefill_f32_workspace_bytes(n, rows, cols, dev->num_cu);
-        if (S % n) ws = std::max(ws, tc::prefill_f32_workspace_bytes(S % n, rows, cols, dev->num_cu));
-    } else {
-        ws = tc::gemm_mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
-    }
-    if (ensure(dev->act, dev->act_bytes, act_bytes) && ensure(dev->aux, dev->aux_bytes, ws)) return true;
-    (void)hipGetLastError();  // the failed allocation's
-    return false;
+    if (recording(st)) return false;
+    size_t act_bytes = 0;
+    const size_t ws = tc::mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
+    return tc::scratch_grow(dev->act, act_bytes, false, false, DeviceMem{}) &&
+           tc::scratch_grow(dev->aux, ws, false, false, DeviceMem{});
 }
 
 // The matrix-core product of a call that route_mfma took.
 int run_mfma(Device *dev, int type, const void *w, const float *x, float *out, uint32_t S, uint32_t rows, uint32_t cols,
              hipStream_t st) {
     if (!tc::prefill_f32_type(type))
-        return tc::gemm_mfma_into(type, w, x, out, S, rows, cols, dev->num_cu, dev->act, dev->aux, st);
-    const uint32_t chunk = gemm_f32_chunk(cols);
+        return tc::gemm_mfma_into(type, w, x, out, S, rows, cols, dev->num_cu, dev->act.p, dev->aux.p, st);
+    const uint32_t chunk = tc::gemm_f32_chunk(cols);
     for (uint32_t s0 = 0; s0 < S; s0 += chunk) {
         const hipError_t e = tc::launch_prefill_f32(type, w, x + size_t(s0) * cols, out + size_t(s0) * rows,
-                                                    std::min(chunk, S - s0), rows, cols, dev->num_cu, dev->act, dev->aux, st);
+                                                    std::min(chunk, S - s0), rows, cols, dev->num_cu, dev->act.p, dev->aux.p, st);
         if (e != hipSuccess) return hip_fail(e, "bf16 MFMA GEMM");
     }
     return TC_OK;
@@ -485,9 +502,10 @@ int tc_gemv_q8(int type, const void *w, const void *act, float *out, uint32_t se
 int tc_gemv_reserve(uint32_t cols, uint32_t seq_len) {
     Device *dev = device();
     if (!dev) return fail(TC_E_UNSUPPORTED, "no gfx950 device");
-    size_t need = 0;
-    for (int t : {TC_Q8_0, TC_Q4_K}) need = std::max(need, tc::act_layout(t, seq_len, cols).bytes);
-    if (!ensure(dev->act, dev->act_bytes, need)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", need);
+    size_t act_bytes = 0;
+    const size_t ws = tc::reserve_scratch(seq_len, cols, dev->num_cu, &act_bytes);
+    if (!ensure(dev->act, act_bytes, nullptr)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", act_bytes);
+    if (!ensure(dev->aux, ws, nullptr)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", ws);
     return TC_OK;
 }
 
@@ -527,8 +545,8 @@ int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_le
             // the MFMA kernel's loads need: no padded copies (4001x2880 at
             // 333 tokens: 54.4 -> 38.7 us)
             if ((rc = tc::gemm_mfma_check(type, seq_len, rows, cp))) return rc;
-            if ((rc = gemm_scratch(dev, type, seq_len, rows, cp))) return rc;
-            return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
+            if ((rc = gemm_scratch(dev, type, seq_len, rows, cp, st))) return rc;
+            return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act.p, dev->aux.p, st);
         }
         Padded p;
         if ((rc = pad_q80(dev, w, nullptr, rows, x, seq_len, cols, &p, st))) return rc;
@@ -545,8 +563,8 @@ int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_le
         return run_mfma(dev, type, w, x, out, seq_len, rows, cols, st);
     }
     if ((rc = tc::gemm_mfma_check(type, seq_len, rows, cols))) return rc;
-    if ((rc = gemm_scratch(dev, type, seq_len, rows, cols))) return rc;
-    return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act, dev->aux, st);
+    if ((rc = gemm_scratch(dev, type, seq_len, rows, cols, st))) return rc;
+    return tc::gemm_mfma_into(type, w, x, out, seq_len, rows, cols, dev->num_cu, dev->act.p, dev->aux.p, st);
 }
 
 int tc_gemm_preferred(uint32_t type, uint32_t, uint32_t) { return type_ok(int(type)) ? 1 : 0; }
@@ -575,10 +593,10 @@ int tc_quantize_act(int type, const float *x, uint32_t seq_len, uint32_t cols, i
         cq = p.cols;
     }
     const tc::ActLayout L = tc::act_layout(type, seq_len, cq);
-    if (!ensure(dev->act, dev->act_bytes, L.bytes)) return fail(TC_E_LAUNCH, "hipMalloc failed");
-    hipError_t e = tc::launch_quant_act(type, x, seq_len, cq, L, dev->act, st);
+    if (!ensure(dev->act, L.bytes, st)) return fail(TC_E_LAUNCH, "hipMalloc failed");
+    hipError_t e = tc::launch_quant_act(type, x, seq_len, cq, L, dev->act.p, st);
     if (e != hipSuccess) return hip_fail(e, "activation quantizer");
-    const char *b = static_cast<const char *>(dev->act);
+    const char *b = static_cast<const char *>(dev->act.p);
     e = hipMemcpy2DAsync(qs, cols, b + L.qs_off, cq, cols, seq_len, hipMemcpyDeviceToDevice, st);
     if (e == hipSuccess)
         e = hipMemcpy2DAsync(d, size_t(cols / blk) * 4, b + L.d_off, size_t(cq / blk) * 4, size_t(cols / blk) * 4,
@@ -600,8 +618,8 @@ int tc_block_isums(int type, const void *w, const float *x, int32_t *isums, uint
     // The decode kernel writes the integer sums as a side output; its fp32
     // results land in a scratch row buffer.
     const size_t need = size_t(seq_len) * rows * 4;
-    if (!ensure(dev->aux, dev->aux_bytes, need)) return fail(TC_E_LAUNCH, "hipMalloc failed");
-    return run_gemv(dev, type, w, nullptr, x, nullptr, static_cast<float *>(dev->aux), nullptr, 0, isums, seq_len,
+    if (!ensure(dev->aux, need, st)) return fail(TC_E_LAUNCH, "hipMalloc failed");
+    return run_gemv(dev, type, w, nullptr, x, nullptr, static_cast<float *>(dev->aux.p), nullptr, 0, isums, seq_len,
                     rows, cols, st);
 }
 
@@ -656,8 +674,8 @@ int moe_grouped(Device *dev, const float *x, const int32_t *ids, const float *wt
     const uint32_t nctr =
         std::max(tc::prefill_grouped_counter_words(ntm_max, FF, 2), tc::prefill_grouped_counter_words(ntm_max, H));
     const size_t o_ctr = take(size_t(nctr) * 4);
-    if (!ensure(dev->aux, dev->aux_bytes, off)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", off);
-    char *b = static_cast<char *>(dev->aux);
+    if (!ensure(dev->aux, off, st)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", off);
+    char *b = static_cast<char *>(dev->aux.p);
     int32_t *pos = reinterpret_cast<int32_t *>(b + o_pos);
     uint32_t *srt = reinterpret_cast<uint32_t *>(b + o_srt), *mt = reinterpret_cast<uint32_t *>(b + o_mt);
     uint32_t *ntm = reinterpret_cast<uint32_t *>(b + o_ntm);
@@ -711,10 +729,10 @@ int tc_moe_ffn(const float *x, const int32_t *ids, const float *wts, uint32_t se
     // Scratch: h and u [pairs][ff], per-pair down outputs [pairs][hidden].
     const size_t hb = (npairs * ff * 4 + 255) & ~size_t(255);
     const size_t need = 2 * hb + npairs * hidden * 4;
-    if (!ensure(dev->aux, dev->aux_bytes, need)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", need);
-    float *h = static_cast<float *>(dev->aux);
-    float *u = reinterpret_cast<float *>(static_cast<char *>(dev->aux) + hb);
-    float *y = reinterpret_cast<float *>(static_cast<char *>(dev->aux) + 2 * hb);
+    if (!ensure(dev->aux, need, st)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", need);
+    float *h = static_cast<float *>(dev->aux.p);
+    float *u = reinterpret_cast<float *>(static_cast<char *>(dev->aux.p) + hb);
+    float *y = reinterpret_cast<float *>(static_cast<char *>(dev->aux.p) + 2 * hb);
     const uint64_t gstride = uint64_t(ff) * (hidden / 256) * 144;
     const uint64_t dstride = uint64_t(hidden) * (ff / 256) * 144;
 
@@ -962,11 +980,7 @@ const void *registered_copy(const void *p, size_t bytes) {
     return nullptr;
 }
 
-struct HostScratch {
-    void *p = nullptr;
-    size_t cap = 0;
-};
-HostScratch g_hw, g_hx, g_ho;  // weights / activations / outputs staged for host-pointer calls
+tc::Scratch g_hw, g_hx, g_ho;  // weights / activations / outputs staged for host-pointer calls
 
 }  // namespace
 
@@ -1013,12 +1027,12 @@ int tc_host_matmul(int type, const uint8_t *W, const float *X, uint32_t seq_len,
     std::lock_guard<std::mutex> lk(g_host_mu);
     const void *wd = registered_copy(W, wbytes);
     if (!wd) {
-        if (!ensure(g_hw.p, g_hw.cap, wbytes)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", wbytes);
+        if (!ensure(g_hw, wbytes, nullptr)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", wbytes);
         if (hipMemcpy(g_hw.p, W, wbytes, hipMemcpyHostToDevice) != hipSuccess)
             return fail(TC_E_LAUNCH, "weight copy to device failed");
         wd = g_hw.p;
     }
-    if (!ensure(g_hx.p, g_hx.cap, xbytes) || !ensure(g_ho.p, g_ho.cap, obytes))
+    if (!ensure(g_hx, xbytes, nullptr) || !ensure(g_ho, obytes, nullptr))
         return fail(TC_E_LAUNCH, "hipMalloc failed");
     if (hipMemcpy(g_hx.p, X, xbytes, hipMemcpyHostToDevice) != hipSuccess)
         return fail(TC_E_LAUNCH, "activation copy to device failed");
@@ -1055,12 +1069,12 @@ int tc_host_matmul_f32(const float *W, const float *X, uint32_t seq_len, uint32_
     std::lock_guard<std::mutex> lk(g_host_mu);
     const void *wd = registered_copy(W, wbytes);
     if (!wd) {
-        if (!ensure(g_hw.p, g_hw.cap, wbytes)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", wbytes);
+        if (!ensure(g_hw, wbytes, nullptr)) return fail(TC_E_LAUNCH, "hipMalloc(%zu) failed", wbytes);
         if (hipMemcpy(g_hw.p, W, wbytes, hipMemcpyHostToDevice) != hipSuccess)
             return fail(TC_E_LAUNCH, "weight copy to device failed");
         wd = g_hw.p;
     }
-    if (!ensure(g_hx.p, g_hx.cap, xbytes) || !ensure(g_ho.p, g_ho.cap, obytes))
+    if (!ensure(g_hx, xbytes, nullptr) || !ensure(g_ho, obytes, nullptr))
         return fail(TC_E_LAUNCH, "hipMalloc failed");
     if (hipMemcpy(g_hx.p, X, xbytes, hipMemcpyHostToDevice) != hipSuccess)
         return fail(TC_E_LAUNCH, "activation copy to device failed");

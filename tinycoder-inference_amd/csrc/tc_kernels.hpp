@@ -94,6 +94,10 @@ size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int
 hipError_t launch_prefill(int type, const void *W, const ActView &act, float *out, uint32_t M, uint32_t N,
                           uint32_t K, int num_cu, void *workspace, hipStream_t st);
 
+// A bound on the workspace of either prefill GEMM below for all types, up to M
+// tokens and N rows, at any K.
+size_t prefill_workspace_bound(uint32_t M, uint32_t N, int num_cu);
+
 // Prefill GEMM for the types that take fp32 activations (tc_prefill_f32.hip;
 // IQ4_NL, Q5_0, IQ2_XS): x is split into bf16 pieces in `act`
 // (prefill_f32_act_bytes, below 4 GiB), `workspace` of
@@ -160,6 +164,13 @@ int device_cu_count();
 bool gemm_mfma_addressable(int type, uint32_t S, uint32_t rows, uint32_t cols);
 int gemm_mfma_check(int type, uint32_t S, uint32_t rows, uint32_t cols);
 size_t gemm_mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu, size_t *act_bytes);
+// The same for any matrix-core product (fp32-activation types in chunks of tokens too).
+size_t mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu, size_t *act_bytes);
+// What tc_gemv_reserve reserves: mfma_scratch's largest over all types, up to S
+// tokens, cols columns and kReserveRows rows (the decode kernel's activations
+// are smaller).
+constexpr uint32_t kReserveRows = 1u << 20;
+size_t reserve_scratch(uint32_t S, uint32_t cols, int num_cu, size_t *act_bytes);
 int gemm_mfma_into(int type, const void *w, const float *x, float *out, uint32_t S, uint32_t rows, uint32_t cols,
                    int num_cu, void *act, void *ws, hipStream_t st);
 int gemm_entry_check(int type, const void *w, const float *x, const float *out, uint32_t S, uint32_t rows,

@@ -1561,6 +1561,15 @@ size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int
     return ctr_bytes(g.ntiles) + part + (pf_short_chain(type) && K / 256 > pf_chain(K / 256) ? part / 2 : 0);  // + the sums
 }
 
+size_t prefill_workspace_bound(uint32_t M, uint32_t N, int num_cu) {
+    // Counters: one per tile of at least 128 rows, at least 64 tokens from 33
+    // tokens on. Partials: at most a workgroup per CU, 256 rows (Q8_0 up to 64
+    // tokens: 128 x 64, as much as 256 x 32), and half again for the
+    // short-chain types' sums.
+    const uint32_t tt = M <= 32 ? 32 : M <= 64 ? 64 : 128;
+    const size_t part = size_t(num_cu) * 2 * tt * 256 * 4;
+    return ctr_bytes(uint64_t((M + 63) / 64) * ((uint64_t(N) + 127) / 128)) + part + part / 2;
+}
 hipError_t launch_prefill(int type, const void *W, const ActView &act, float *out, uint32_t M, uint32_t N,
                           uint32_t K, int num_cu, void *workspace, hipStream_t st) {
     const bool ragged = type == kQ8_0 && K % 256 != 0;

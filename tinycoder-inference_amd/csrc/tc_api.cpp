@@ -378,20 +378,22 @@ bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols) {
 
 // Whether a call that the decode kernel could serve goes to the matrix cores;
 // its scratch is in place then. The decode kernel keeps calls of 8 tokens or
-// less but for the above, those that need more than 32-bit offsets or than the
-// memory left, and those under graph capture, which it serves from less
-// scratch or none (the MFMA path's could not grow there, and its address would
-// be held by the graph).
+// less but for the above, and those that need more than 32-bit offsets or than
+// the memory left. A call that is being recorded into a graph goes the same way
+// as outside (so replays give the eager call's bits) where the scratch is in
+// place, by tc_gemv_reserve or an earlier call; it cannot grow there, and the
+// decode kernel needs less or none.
 bool route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
     const bool f32 = tc::prefill_f32_type(type);
     if ((S <= 8 && !few_tokens_mfma(type, S, rows, cols)) || !(f32 || tc::prefill_type(type)) ||
         !tc::gemm_mfma_addressable(type, S, rows, cols))
         return false;
-    if (recording(st)) return false;
     size_t act_bytes = 0;
     const size_t ws = tc::mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);
-    return tc::scratch_grow(dev->act, act_bytes, false, false, DeviceMem{}) &&
-           tc::scratch_grow(dev->aux, ws, false, false, DeviceMem{});
+    const bool rec = recording(st);
+    if (rec && (dev->act.bytes < act_bytes || dev->aux.bytes < ws)) return false;
+    return tc::scratch_grow(dev->act, act_bytes, rec, false, DeviceMem{}) &&
+           tc::scratch_grow(dev->aux, ws, rec, false, DeviceMem{});
 }
 
 // The matrix-core product of a call that route_mfma took.

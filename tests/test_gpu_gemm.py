@@ -205,7 +205,44 @@ def test_few_tokens_on_the_matrix_cores(tc, dev, oracle, qt, S, N, K):
         assert np.array_equal(out.cpu().numpy(), got), NAMES[qt]
 
 
+# Byte offsets of the fp16 scales of a block.
+SCALES = {Q8_0: (0,), Q2_K: (80, 82), Q3_K: (108,), Q4_K: (0, 2), Q5_K: (0, 2), Q6_K: (208,)}
+
+
+def even_blocks(qt, rng, rows, cols, scale=2.0**-10):
+    """Random blocks whose scales lie within a factor of 3, so that every
+    superblock counts alike in a sum."""
+    from qdata import TYPE_SIZE
+    b = random_blocks(qt, rng, rows, cols).reshape(-1, TYPE_SIZE[qt])
+    for o in SCALES.get(qt, (0,)):
+        b[:, o:o + 2] = rng.uniform(scale, 3 * scale, len(b)).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    return b.ravel()
+
+
 LOW = [Q2_K, Q3_K, IQ4_XS, IQ4_NL, Q5_0, IQ2_XS]
+
+
+@pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ4_XS])
+def test_gemm_low_bit_overflow(tc, dev, oracle, qt):
+    """Activations so large that block values overflow: infinities of their
+    sign, also where a workgroup has more superblocks than one chain of sums
+    holds (256 whole tiles of 14 superblocks), and no NaN."""
+    rng = np.random.default_rng(qt + 31)
+    M, N, K = 1024, 8192, 3584
+    w = even_blocks(qt, rng, N, K, 2.0**(-12 if qt == IQ4_XS else -6))
+    x = gaussian(rng, (M, K))
+    x[3] = 0.0
+    x[3, :256] = gaussian(rng, 256) * np.float32(1e38)
+    got = tc.gemm(qt, to_dev(w, dev), to_dev(x, dev), N, K).cpu().numpy()[3]
+    wr = w.reshape(N, -1)[:, :row_bytes(qt, 256)]
+    qs, d, _ = oracle.quantize_q8k(x[3, :256])
+    ref = oracle.dequant(qt, np.ascontiguousarray(wr), N, 256).astype(np.float64) @ (qs.astype(np.float64).ravel() * float(d[0]))
+    top = float(np.finfo(np.float32).max)
+    over = np.abs(ref) > 1.01 * top
+    under = np.abs(ref) < 0.99 * top
+    assert over.sum() > 100 and under.sum() > 100
+    assert (got[over] == np.sign(ref[over]) * np.inf).all(), got[over][:8]
+    assert np.allclose(got[under], ref[under], rtol=1e-4, atol=1e-6 * top)
 
 
 @pytest.mark.parametrize("qt", LOW)

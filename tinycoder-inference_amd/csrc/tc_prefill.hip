@@ -1132,7 +1132,8 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const float s = p[r] + acc[t][r];
-                    acc[t][r] = back ? s : acc[t][r] - (s - p[r]);
+                    // (an infinite or NaN sum has no rounding: it would leave NaN)
+                    acc[t][r] = back ? s : __builtin_isfinite(s) ? acc[t][r] - (s - p[r]) : 0.0f;
                     if (!back) fl[(16 * t + r) * 512] = s;
                 }
             }

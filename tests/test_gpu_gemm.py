@@ -219,6 +219,37 @@ def even_blocks(qt, rng, rows, cols, scale=2.0**-10):
     return b.ravel()
 
 
+# (20000 x 18944: tiles split over 3 workgroups; 21000 x 8192: the same with 11
+# superblocks each; 10496 x 18944: over more workgroups, 12 superblocks each)
+@pytest.mark.parametrize("N,K", [(20000, 18944), (21000, 8192), (10496, 18944)])
+@pytest.mark.parametrize("qt", [t for t in MFMA_TYPES if t != Q8_0])
+def test_sums_as_close_as_the_decode_kernels(tc, dev, oracle, qt, N, K):
+    """Where the decode kernel could serve a call, the fp32 sums of the
+    matrix-core kernels are no further from the 64-bit results (2-norm) than its
+    own (single tokens, which always run it)."""
+    import torch
+    rng = np.random.default_rng(N + K + qt)
+    w = even_blocks(qt, rng, N, K)
+    S = 8 if qt in MFMA_TYPES else 9
+    x = gaussian(rng, (S, K))
+    wd, xd = to_dev(w, dev), to_dev(x, dev)
+    got = tc.gemv(qt, wd, xd, N, K) if S <= 8 else tc.gemm(qt, wd, xd, N, K)
+    dec = torch.cat([tc.gemv(qt, wd, xd[s:s + 1].contiguous(), N, K) for s in range(S)])
+    rows = np.sort(rng.choice(N, 4000, replace=False))
+    if qt in (IQ2_XS, IQ4_NL, Q5_0):
+        xa = x.astype(np.float64)
+    else:
+        qs, d, _ = oracle.quantize_q8k(x.ravel())
+        xa = (qs.reshape(-1, 256).astype(np.float64) * d.reshape(-1, 1).astype(np.float64)).reshape(S, K)
+    # (products of an fp16 scale, a 4 to 8 bit scale and a quant are exact in
+    # fp32, or nearly: Q6_K, and the mins of Q2_K, Q4_K and Q5_K)
+    ref = xa @ oracle.dequant(qt, w.reshape(N, -1)[rows], len(rows), K).astype(np.float64).T
+    err = [np.linalg.norm(o.cpu().numpy()[:, rows] - ref) / np.linalg.norm(ref) for o in (got, dec)]
+    print(f"{NAMES[qt]} {N}x{K}: {err[0]:.3e}, decode kernel {err[1]:.3e}")
+    # (the norms over 4000 rows scatter by below 1%)
+    assert err[0] <= 1.02 * err[1], (NAMES[qt], N, K, err)
+
+
 LOW = [Q2_K, Q3_K, IQ4_XS, IQ4_NL, Q5_0, IQ2_XS]
 
 

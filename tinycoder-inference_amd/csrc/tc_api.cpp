@@ -362,12 +362,11 @@ int gemm_batched(Device *dev, int type, const void *w, const float *x, float *ou
 // tokens 21 / 28, 5 tokens 35 / 28; at 64 MB two decode launches' streams take
 // as long as the MFMA kernel's one). The fp32-activation types also where their
 // 512-thread launch no longer fits (18944x3584: IQ4_NL 4 tokens 49 / 37, 5
-// tokens 108 / 38; Q5_0 46 / 41; IQ2_XS 5 tokens 44 / 41).
-bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols) {
+// tokens 108 / 38; Q5_0 46 / 41; IQ2_XS 5 tokens 44 / 41). Only where the sums
+// are no further from the 64-bit results than the decode kernel's.
+bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu) {
     const uint32_t smax = tc::gemv_max_tokens(type, cols);
-    // (Q8_0's MFMA sums of 32-wide blocks are further from the 64-bit results
-    // than the decode kernel's: 1.6e-7 against 0.9e-7 at 18944 columns)
-    if (smax == 0 || type == TC_Q8_0) return false;
+    if (smax == 0 || !(tc::prefill_f32_type(type) || tc::prefill_short_sums(type, S, rows, cols, num_cu))) return false;
     const uint32_t launches = (S + smax - 1) / smax;
     const uint64_t bytes = uint64_t(rows) * tc_row_bytes(type, cols);
     if (launches >= (tc::prefill_f32_type(type) && bytes < (16u << 20) ? 5u : 3u)) return true;
@@ -385,7 +384,7 @@ bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols) {
 // decode kernel needs less or none.
 bool route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
     const bool f32 = tc::prefill_f32_type(type);
-    if ((S <= 8 && !few_tokens_mfma(type, S, rows, cols)) || !(f32 || tc::prefill_type(type)) ||
+    if ((S <= 8 && !few_tokens_mfma(type, S, rows, cols, dev->num_cu)) || !(f32 || tc::prefill_type(type)) ||
         !tc::gemm_mfma_addressable(type, S, rows, cols))
         return false;
     size_t act_bytes = 0;

@@ -94,6 +94,8 @@ size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int
 hipError_t launch_prefill(int type, const void *W, const ActView &act, float *out, uint32_t M, uint32_t N,
                           uint32_t K, int num_cu, void *workspace, hipStream_t st);
 
+// Whether a launch's fp32 sums are as short as the decode kernel's.
+bool prefill_short_sums(int type, uint32_t M, uint32_t N, uint32_t K, int num_cu);
 // A bound on the workspace of either prefill GEMM below for all types, up to M
 // tokens and N rows, at any K.
 size_t prefill_workspace_bound(uint32_t M, uint32_t N, int num_cu);

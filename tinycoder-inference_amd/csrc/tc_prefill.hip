@@ -1562,6 +1562,22 @@ size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int
     return ctr_bytes(g.ntiles) + part + (pf_short_chain(type) && K / 256 > pf_chain(K / 256) ? part / 2 : 0);  // + the sums
 }
 
+// The decode kernel adds a row's superblock values in a tree; a workgroup here
+// adds them one after the other, up to units / G of them, and where tiles are
+// not summed in fp64 (the fixup launch) the parts too in fp32. Error (2-norm,
+// 1e-8) at 8 tokens, decode kernel against this one: Q6_K 18432x8192 (9 per
+// workgroup) 7.1 / 6.5, 10496x18944 (12) 7.9 / 7.3, but 20480x8192 (10, summed
+// in the kernel) 7.1 / 7.5, 20000x18944 (24, likewise) 7.9 / 10.1, 18944x18944
+// (21, fixup) 7.9 / 8.8, 65536x8192 (whole tiles of 32) 7.1 / 10.6; Q4_K and the
+// IQ types alike. Q8_0's sums of 32-wide blocks are longer: 9 against 16 at
+// 18944 columns. The short-chain types hold it at any length.
+bool prefill_short_sums(int type, uint32_t M, uint32_t N, uint32_t K, int num_cu) {
+    if (!prefill_type(type) || type == kQ8_0) return false;
+    if (pf_short_chain(type)) return true;
+    const PfGeom g = pf_geom(type, M, N, K, num_cu);
+    const uint64_t units = uint64_t(g.ntiles) * (K / 256);
+    return !g.fused && units <= uint64_t(g.G) * (K / 256 <= 48 ? 9 : 12);
+}
 size_t prefill_workspace_bound(uint32_t M, uint32_t N, int num_cu) {
     // Counters: one per tile of at least 128 rows, at least 64 tokens from 33
     // tokens on. Partials: at most a workgroup per CU, 256 rows (Q8_0 up to 64

@@ -52,7 +52,7 @@ int tc_available(void);
 
 /* Decode mat-vec, seq_len 1..8: out[s][r] = x[s] . W[r]. Several tokens whose
  * activations do not fit one launch of the decode kernel go through tc_gemm's
- * kernels (under stream capture: where the scratch is in place, by
+ * kernels where those are faster and as accurate (under stream capture: where the scratch is in place, by
  * tc_gemv_reserve or an earlier call; else by the decode kernel).
  * Replaces tinycoder::gpu::int8Gemv (include/Int8Gemm.hpp:77-78,
  * src/cpp/core/cuda/gemm/GemmDispatch.cu:788). cols % 256 == 0. */
@@ -101,8 +101,9 @@ int tc_gemv_dual(int type, const void *wg, const void *wu, const float *x, float
  * (Q4_K, Q5_K, Q6_K, Q8_0, IQ3_XXS, IQ3_S, IQ2_S; GemmDispatch.cu:600-602)
  * and, from 9 tokens on, for Q2_K, Q3_K and IQ4_XS; bf16 MFMA on x split into
  * three pieces, from 9 tokens on, for IQ2_XS, IQ4_NL and Q5_0. Up to 8 tokens
- * those six go as tc_gemv; under stream capture without the scratch in place
- * they run the decode kernel over groups of 8 tokens.
+ * those six go as tc_gemv; some of 9 to 13 tokens that it serves faster, and
+ * calls under stream capture without the scratch in place, run the decode
+ * kernel over groups of 8 tokens.
  * blocks_per_row must equal cols / block_elems. */
 int tc_gemm(int type, const void *w, const float *x, float *out, uint32_t seq_len, uint32_t rows,
             uint32_t cols, uint32_t blocks_per_row, void *stream);

@@ -246,3 +246,42 @@ int main() {
     return 0;
 }
 """)
+
+
+def test_route_by_measured_times(tmp_path):
+    """Calls of few tokens that the decode kernel was measured to serve faster
+    keep it, and the gains of the matrix-core route stay (times in us, decode
+    kernel against matrix cores)."""
+    import tc_hip
+    few = [("Q5_0", 4, 18944, 2048, 18, 30), ("Q5_0", 5, 18944, 2048, 20, 30), ("Q5_0", 4, 8192, 4096, 19, 28),
+           ("Q5_0", 6, 32768, 1536, 23, 30), ("Q5_0", 2, 2560, 14336, 23, 34), ("IQ4_NL", 2, 3584, 13824, 21, 30),
+           ("IQ4_NL", 4, 8192, 4096, 22, 27), ("IQ2_XS", 5, 32768, 3072, 37, 45), ("Q6_K", 2, 2560, 14336, 20, 27),
+           ("Q6_K", 4, 2560, 8192, 21, 24), ("Q5_K", 6, 5120, 8192, 19, 24), ("Q5_K", 8, 3584, 10240, 24, 25),
+           ("Q4_K", 4, 2560, 18944, 18, 23), ("IQ4_XS", 5, 3584, 13824, 21, 26), ("IQ4_XS", 6, 5120, 10240, 26, 28),
+           ("Q6_K", 8, 3584, 18944, 137, 33), ("Q4_K", 8, 3584, 18944, 45, 26), ("IQ4_NL", 8, 3584, 18944, 163, 41),
+           ("IQ4_NL", 5, 18944, 3584, 108, 38), ("Q6_K", 3, 256, 18944, 33, 21), ("Q5_K", 7, 5120, 11008, 36, 24)]
+    prompt = [("IQ4_XS", 9, 8192, 2048, 15, 19), ("IQ4_XS", 9, 8192, 4096, 21, 27), ("IQ4_XS", 11, 4096, 1280, 14, 16),
+              ("Q2_K", 9, 4096, 4096, 16, 17), ("IQ2_XS", 9, 8192, 2048, 22, 27), ("IQ4_XS", 9, 8192, 512, 13, 11),
+              ("IQ4_XS", 14, 4096, 2560, 20, 16), ("IQ4_XS", 9, 12288, 3072, 27, 23), ("Q2_K", 9, 256, 256, 14, 8),
+              ("Q2_K", 10, 4096, 4096, 18, 17), ("IQ2_XS", 9, 7168, 2304, 45, 24), ("Q5_0", 9, 18944, 3584, 150, 40)]
+    rows = [f"{{{int(f is few)}, {tc_hip.TYPES[t]}, {s}, {n}, {k}, {int(mf < dec)}}}"
+            for f in (few, prompt) for t, s, n, k, dec, mf in f]
+    _compile_and_run(tmp_path, r"""
+#include <stdint.h>
+#include <stdio.h>
+namespace tc {
+bool few_tokens_mfma(int, uint32_t, uint32_t, uint32_t, int);
+bool prompt_mfma(int, uint32_t, uint32_t, uint32_t);
+}
+int main() {
+    const uint32_t c[][6] = {""" + ", ".join(rows) + r"""};
+    for (auto &r : c) {
+        const bool m = r[0] ? tc::few_tokens_mfma(int(r[1]), r[2], r[3], r[4], 256)
+                            : tc::prompt_mfma(int(r[1]), r[2], r[3], r[4]);
+        if (m == bool(r[5])) continue;
+        printf("type %u, %u tokens, %u x %u: matrix cores %d\n", r[1], r[2], r[3], r[4], int(m));
+        return 1;
+    }
+    return 0;
+}
+""")

@@ -318,6 +318,78 @@ size_t mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_
     return ws;
 }
 
+namespace {
+bool few_tokens_faster(int type, uint32_t S, uint32_t rows, uint32_t cols) {
+    const bool f32 = prefill_f32_type(type);
+    const uint32_t smax = gemv_max_tokens(type, cols);
+    if (smax == 0 || type == TC_Q8_0 || (!f32 && smax >= S)) return false;
+    const uint32_t launches = (S + smax - 1) / smax;
+    const uint64_t bytes = uint64_t(rows) * tc_row_bytes(type, cols);
+    auto mb = [](uint64_t n) { return n << 20; };
+    if (bytes < mb(16)) {
+        // (256 rows: 21 against 33 us and more; IQ4_NL 1024x16384 in 5 launches
+        // 34 / 41, Q5_K 5 tokens in 3 24 / 26)
+        if (f32) return launches >= (bytes >= mb(12) ? 5u : 6u);
+        return launches >= 3 && (type != TC_Q5_K || S >= 6);
+    }
+    if (launches >= 3) return true;  // (Q6_K 3584x18944 8 tokens 137 / 33)
+    if (bytes > mb(64)) return false;
+    if (launches == 2) switch (type) {
+            // (2560x18944 4 tokens 18 / 23, 5120x11008 7 tokens .61 of the
+            // decode kernel's time, 5120x13824 5 tokens .67)
+            case TC_Q4_K:
+            case TC_IQ4_XS: return S >= 7 || (S >= 5 && bytes >= mb(36));
+            // (3584x10240 8 tokens 24 / 25, 5120x11008 6 tokens .72)
+            case TC_Q5_K: return S >= 6 && bytes >= mb(36);
+            // (2560x8192 4 tokens 21 / 24, 5120x11008 .81)
+            case TC_Q6_K: return S >= 5 || (S == 4 && bytes >= mb(26));
+            // (3584x13824 2 tokens 21 / 30; 4 tokens 2560x12288 26 / 28, 3584x11008 .85)
+            case TC_IQ4_NL:
+            case TC_Q5_0: return S >= 5 || (S == 4 && bytes >= mb(21));
+            default: return S >= 4;  // (.38 to .96)
+        }
+    // one launch, which for the fp32-activation types is slow where it takes
+    // the smaller workgroup (18944x3584 5 tokens: IQ4_NL 108 / 38)
+    switch (type) {
+        case TC_IQ4_NL: return S >= 5 || (S == 4 && bytes >= mb(24));                  // (8192x4096 4 tokens 22 / 27)
+        case TC_Q5_0: return S >= 7 || (S == 6 && cols >= 3584);                       // (18944x2048 5 tokens 20 / 30)
+        case TC_IQ2_XS: return S >= 6 || (S == 5 && cols >= 3584);                     // (32768x3072 5 tokens 37 / 45)
+        default: return false;
+    }
+}
+}  // namespace
+
+bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu) {
+    return few_tokens_faster(type, S, rows, cols) &&
+           (prefill_f32_type(type) || prefill_short_sums(type, S, rows, cols, num_cu));
+}
+
+bool prompt_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols) {
+    if (!prefill_f32_type(type) && !prefill_type(type)) return false;
+    const uint32_t nblk = cols / 256;
+    const uint64_t units = uint64_t(rows) * nblk;
+    // the decode kernel's passes over the matrix, 65536 superblocks each, and
+    // whether the last is at least two thirds full
+    const uint64_t passes = (units + 65535) / 65536;
+    const bool full = units >= (passes - 1) * 65536 + 43690;
+    if (passes > 2) return true;
+    switch (type) {
+        // (9 tokens: 8192x1280 13.5 / 16.9, 8192x2048 15.5 / 19.2, 8192x4096 21.3
+        // / 26.6, 4096x2560 1.08 and 3072x5120 1.11 of the decode kernel's time;
+        // 12 tokens: 8192x2048 1.08, 4096x3584 .88)
+        case TC_IQ4_XS:
+            if (nblk < 3) return true;
+            if (nblk % 4 == 0 && nblk <= 16 && full && S <= (passes == 1 ? 12u : 11u)) return false;
+            return passes > 1 || S > (nblk == 3 || nblk == 5 ? 13u : nblk <= 16 ? 11u : nblk <= 24 ? 9u : 8u);
+        // (9 tokens of 4096 columns: 4096 rows 15.6 / 16.9, 8192 rows 22.1 / 24.2)
+        case TC_Q2_K:
+        case TC_Q3_K: return !(S == 9 && nblk == 16 && full);
+        // (9 tokens: 8192x2048 22.5 / 27.0, 5120x3072 22.6 / 25.2; 13: 1.0)
+        case TC_IQ2_XS: return !(S <= 11 && passes == 1 && full && nblk % 2 == 0 && nblk <= 14);
+        default: return true;
+    }
+}
+
 size_t reserve_scratch(uint32_t S, uint32_t cols, int num_cu, size_t *act_bytes) {
     *act_bytes = 0;
     if (S == 0 || cols == 0) return 0;
@@ -352,40 +424,16 @@ int gemm_batched(Device *dev, int type, const void *w, const float *x, float *ou
     return TC_OK;
 }
 
-// Whether up to 8 tokens go to the matrix cores rather than to the decode
-// kernel, which takes smax tokens per launch (its LDS holds their activations)
-// and reads the weights once per launch: from 3 launches on (small matrices of
-// the fp32-activation types from 5), and from 2 where that measured faster (us,
-// decode against MFMA: Q6_K 3584x18944 3 tokens 51 / 33, 8 tokens 137 / 33,
-// 256x18944 33 / 21 and 87 / 21; Q4_K 3584x18944 4 tokens 26 / 26, 8 tokens 45
-// / 26; Q5_K 3 tokens 28 / 32, 5000x9216 5 tokens 23 / 26; IQ4_NL 256x18944 3
-// tokens 21 / 28, 5 tokens 35 / 28; at 64 MB two decode launches' streams take
-// as long as the MFMA kernel's one). The fp32-activation types also where their
-// 512-thread launch no longer fits (18944x3584: IQ4_NL 4 tokens 49 / 37, 5
-// tokens 108 / 38; Q5_0 46 / 41; IQ2_XS 5 tokens 44 / 41). Only where the sums
-// are no further from the 64-bit results than the decode kernel's.
-bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu) {
-    const uint32_t smax = tc::gemv_max_tokens(type, cols);
-    if (smax == 0 || !(tc::prefill_f32_type(type) || tc::prefill_short_sums(type, S, rows, cols, num_cu))) return false;
-    const uint32_t launches = (S + smax - 1) / smax;
-    const uint64_t bytes = uint64_t(rows) * tc_row_bytes(type, cols);
-    if (launches >= (tc::prefill_f32_type(type) && bytes < (16u << 20) ? 5u : 3u)) return true;
-    if (bytes < (16u << 20) || bytes > (64u << 20)) return false;
-    if (launches == 2 && S >= (smax == 1 ? 2u : type == TC_Q5_K ? 6u : 4u)) return true;
-    return tc::prefill_f32_type(type) && S >= (type == TC_IQ2_XS ? 5u : 4u);
-}
-
 // Whether a call that the decode kernel could serve goes to the matrix cores;
-// its scratch is in place then. The decode kernel keeps calls of 8 tokens or
-// less but for the above, and those that need more than 32-bit offsets or than
-// the memory left. A call that is being recorded into a graph goes the same way
+// its scratch is in place then. The decode kernel keeps those that it serves
+// faster (few_tokens_mfma, prompt_mfma) and those that need more than 32-bit
+// offsets or than the memory left. A call that is being recorded into a graph goes the same way
 // as outside (so replays give the eager call's bits) where the scratch is in
 // place, by tc_gemv_reserve or an earlier call; it cannot grow there, and the
 // decode kernel needs less or none.
 bool route_mfma(Device *dev, int type, uint32_t S, uint32_t rows, uint32_t cols, hipStream_t st) {
-    const bool f32 = tc::prefill_f32_type(type);
-    if ((S <= 8 && !few_tokens_mfma(type, S, rows, cols, dev->num_cu)) || !(f32 || tc::prefill_type(type)) ||
-        !tc::gemm_mfma_addressable(type, S, rows, cols))
+    if (!tc::gemm_mfma_addressable(type, S, rows, cols) ||
+        !(S <= 8 ? tc::few_tokens_mfma(type, S, rows, cols, dev->num_cu) : tc::prompt_mfma(type, S, rows, cols)))
         return false;
     size_t act_bytes = 0;
     const size_t ws = tc::mfma_scratch(type, S, rows, cols, dev->num_cu, &act_bytes);

@@ -193,20 +193,17 @@ uint32_t gemv_fused_quant_limit(int type, uint64_t weight_bytes) {
 }
 
 uint32_t gemv_max_tokens(int type, uint32_t cols) {
-    uint32_t best = 0;
-    if (tiled_type(type)) {
-        for (uint32_t S = 1; S <= 8; ++S) {
-            TLaunchArgs a;
-            const uint32_t f = std::max(tlds_layout<CfgBig>(type, S, cols, &a), tlds_layout<CfgSmall>(type, S, cols, &a));
-            // Q8_0 and (when the 512-thread shape does not fit) the fp32
-            // activation types launch the 256-thread shape only
-            const bool small_only = type == kQ8_0 || fp32_act_type(type);
-            if ((small_only ? tlds_layout<CfgSmall>(type, S, cols, &a) : f) + 2 * 8 * S * (cols / 256) * 4 <=
-                kTLdsBudget)
-                best = S;
-        }
+    if (!tiled_type(type)) return 0;
+    for (uint32_t S = 8; S >= 1; --S) {  // (from 8 down: narrow inputs, the small calls, end at once)
+        TLaunchArgs a;
+        const uint32_t f = std::max(tlds_layout<CfgBig>(type, S, cols, &a), tlds_layout<CfgSmall>(type, S, cols, &a));
+        // Q8_0 and (when the 512-thread shape does not fit) the fp32
+        // activation types launch the 256-thread shape only
+        const bool small_only = type == kQ8_0 || fp32_act_type(type);
+        if ((small_only ? tlds_layout<CfgSmall>(type, S, cols, &a) : f) + 2 * 8 * S * (cols / 256) * 4 <= kTLdsBudget)
+            return S;
     }
-    return best;
+    return 0;
 }
 
 hipError_t launch_gemv_jobs(int type, uint32_t S, const GemvJob *jobs, uint32_t njobs, int num_cu,

@@ -168,6 +168,18 @@ int gemm_mfma_check(int type, uint32_t S, uint32_t rows, uint32_t cols);
 size_t gemm_mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu, size_t *act_bytes);
 // The same for any matrix-core product (fp32-activation types in chunks of tokens too).
 size_t mfma_scratch(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu, size_t *act_bytes);
+// Whether tc_gemv's 2 to 8 tokens go to the matrix cores. The decode kernel
+// takes gemv_max_tokens per launch (its LDS holds their activations) and reads
+// the weights once per launch, so it loses where it needs several; the rule is
+// drawn from all shapes of 256 to 32768 rows and 1024 to 18944 columns
+// measured both ways, and takes none that it would slow down by over 2.5%. Only
+// where the sums are no further from the 64-bit results than its own.
+bool few_tokens_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols, int num_cu);
+// Whether tc_gemm's 9 tokens or more of the types that the decode kernel
+// could serve (over groups of 8) go to the matrix cores: all but 9 to 13 of a
+// few types on matrices that two of its launches get through in one or two
+// full passes.
+bool prompt_mfma(int type, uint32_t S, uint32_t rows, uint32_t cols);
 // What tc_gemv_reserve reserves: mfma_scratch's largest over all types, up to S
 // tokens, cols columns and kReserveRows rows (the decode kernel's activations
 // are smaller).

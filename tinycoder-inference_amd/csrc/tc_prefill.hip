@@ -181,8 +181,11 @@ __host__ __device__ constexpr uint32_t pf_grid_bytes(int type) {
 // accumulators, which then go into fp32 sums in memory, their rounding staying
 // behind in the accumulators (one fp32 chain over all of K was further from
 // the 64-bit results than the decode kernel's tree: Q3_K 3584x18944 M = 2048
-// 1.28e-7 against 0.79e-7, now 0.78e-7; 299 us instead of 270).
-__host__ __device__ constexpr uint32_t pf_chain(uint32_t nblk) { return nblk <= 48 ? 8 : 12; }
+// 1.28e-7 against 0.79e-7, now 0.78e-7; 299 us instead of 270). Long rows take
+// 12, but 9 where the fp32 partials of 3 workgroups or more are added up (Q3_K
+// 20000x18944 M = 100: 0.82e-7 with 12, 0.76e-7 with 9, 0.74e-7 with 8, decode
+// kernel 0.78e-7; 106, 111 and 115 us: every flush of all workgroups moves 60 MB).
+__host__ __device__ constexpr uint32_t pf_chain(uint32_t nblk, bool parts) { return nblk <= 48 ? 8 : parts ? 9 : 12; }
 __host__ __device__ constexpr bool pf_short_chain(int type) { return type == kQ2_K || type == kQ3_K || type == kIQ4_XS; }
 template <int TYPE, int NT>
 constexpr bool pf_shared_w() { return ((TYPE == kQ5_K || TYPE == kQ6_K) && NT == 4) || TYPE == kQ8W || TYPE == kQ8RW; }
@@ -1120,15 +1123,26 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         // Short chains: the accumulators into the thread's sums (behind the
         // partial tiles, value r of token block t at (16 t + r) * 512 + the
         // thread), or the sums back into them.
+        const uint32_t chain = pf_chain(a.nblk, a.fused && 3 * a.ntiles <= 2 * a.G);
         uint32_t held = 0;     // superblocks in acc
         bool flushed = false;  // earlier ones are in the sums
         auto spill = [&](bool back) __attribute__((always_inline)) {
             float *const fl = a.ws + size_t(a.G) * 2 * (TT * PR) + size_t(v) * (TT * PR) + (64 * w + lane_now());
+            if (!back && !flushed) {  // (the sums start from 0)
+#pragma unroll
+                for (int t = 0; t < NB; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        fl[(16 * t + r) * 512] = acc[t][r];
+                        acc[t][r] = 0.0f;
+                    }
+                return;
+            }
 #pragma unroll
             for (int t = 0; t < NB; ++t) {
                 float p[16];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) p[r] = flushed ? fl[(16 * t + r) * 512] : 0.0f;
+                for (int r = 0; r < 16; ++r) p[r] = fl[(16 * t + r) * 512];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const float s = p[r] + acc[t][r];
@@ -1297,7 +1311,7 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             __builtin_amdgcn_sched_barrier(0);
             ph ^= 1;
             if constexpr (pf_short_chain(TYPE)) {
-                if (++held == pf_chain(a.nblk) && b + 1 < b1) {
+                if (++held == chain && b + 1 < b1) {
                     spill(false);
                     held = 0;
                     flushed = true;
@@ -1374,28 +1388,53 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const bool last = *flag == ncontrib - 1;  // the counter wrapped back to 0
         if (!last) continue;
         const uint32_t first_slot = sk_begin(units, a.G, vf) < t0 ? 1u : 0u;  // vf's second segment
-        // this lane's partial of contributor c, into p
-        auto ld = [&](uint32_t c, float (&p)[NB][16]) __attribute__((always_inline)) {
+        // this lane's partial of contributor c, the token blocks of p from tb on
+        auto ld = [&](uint32_t c, int tb, auto &p) __attribute__((always_inline)) {
             const float *src = a.ws + (size_t(c) * 2 + (c == vf ? first_slot : 0u)) * (TT * PR);
             uint32_t lo = 4 * g * PR + rl;  // this lane's offset, recomputed per contributor
             asm volatile("" : "+v"(lo));
 #pragma unroll
-            for (int t = 0; t < NB; ++t)
+            for (int t = 0; t < int(sizeof(p) / sizeof(p[0])); ++t)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        p[t][4 * q + e] = __hip_atomic_load(src + (32 * (tg * NB + t) + 8 * q + e) * PR + lo,
+                        p[t][4 * q + e] = __hip_atomic_load(src + (32 * (tg * NB + tb + t) + 8 * q + e) * PR + lo,
                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         };
         if (ncontrib == 2) {
             // own + other in either order: the same bits
             float p[NB][16];
-            ld(other, p);
+            ld(other, 0, p);
 #pragma unroll
             for (int t = 0; t < NB; ++t)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[t][r] += p[t][r];
+        } else if (pf_short_chain(TYPE) && a.nblk > 20) {
+            // as below, but two at a time and these pairs in range order: an
+            // addition less per value of 4 partials (Q3_K 8192x8192 M = 200: 0.718e-7
+            // -> 0.705e-7, decode kernel 0.705e-7). Half of a 128-token tile at a
+            // time, which the registers hold. (Shorter rows are closer than the
+            // decode kernel without, and this costs 1.3 us at 5 partials.)
+            constexpr int NH = NB == 4 ? 2 : NB;
+#pragma unroll
+            for (int tb = 0; tb < NB; tb += NH)
+                for (uint32_t c = vf; c <= vl; c += 2) {
+                    float s[NH][16], p[NH][16];
+                    ld(c, tb, s);
+                    if (c < vl) {
+                        ld(c + 1, tb, p);
+#pragma unroll
+                        for (int t = 0; t < NH; ++t)
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) s[t][r] += p[t][r];
+                    }
+#pragma unroll
+                    for (int t = 0; t < NH; ++t)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            acc[tb + t][r] = c == vf ? s[t][r] : acc[tb + t][r] + s[t][r];
+                }
         } else {
             // every contributor's partial from memory in range order (this
             // workgroup's too: it is there already, and acc's registers then
@@ -1403,7 +1442,7 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             for (uint32_t c = vf; c <= vl; ++c) {
                 if (!live(c)) continue;
                 float p[NB][16];
-                ld(c, p);
+                ld(c, 0, p);
 #pragma unroll
                 for (int t = 0; t < NB; ++t)
 #pragma unroll
@@ -1559,7 +1598,7 @@ size_t prefill_workspace_bytes(int type, uint32_t M, uint32_t N, uint32_t K, int
     if (!prefill_type(type)) return 0;
     const PfGeom g = pf_geom(type, M, N, K, num_cu);
     const size_t part = size_t(g.G) * 2 * g.tt * g.pr * 4;
-    return ctr_bytes(g.ntiles) + part + (pf_short_chain(type) && K / 256 > pf_chain(K / 256) ? part / 2 : 0);  // + the sums
+    return ctr_bytes(g.ntiles) + part + (pf_short_chain(type) && K / 256 > pf_chain(K / 256, true) ? part / 2 : 0);  // + the sums
 }
 
 // The decode kernel adds a row's superblock values in a tree; a workgroup here

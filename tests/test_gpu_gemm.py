@@ -112,8 +112,8 @@ def test_gemm_low_bit_mfma(tc, dev, oracle, qt, M, N, K):
 
 # The fp32-activation types on the bf16 matrix cores (x as three exact bf16
 # pieces): from 9 tokens, tile edges and remainders, an odd number of 74-byte
-# units, split tiles, a tile kept whole over 9 superblocks ((300, 7000, 2304):
-# more tiles than workgroups), activations over 12 orders of magnitude.
+# units, split tiles ((300, 7000, 2304): 84 over 256 workgroups, whole ones at
+# 256 columns), activations over 12 orders of magnitude.
 # Every product is exact; the fp32 sums of K / 32 block sums, each of at
 # most 12 roundings, stay within (K / 32 + 12) 2^-24 |x| . |w| of the exact
 # value here and in the oracle.
@@ -253,6 +253,36 @@ def test_sums_as_close_as_the_decode_kernels(tc, dev, oracle, qt, S, N, K):
 
 
 LOW = [Q2_K, Q3_K, IQ4_XS, IQ4_NL, Q5_0, IQ2_XS]
+
+
+# Units (tile, superblock) per workgroup of 256, chains of 8 superblocks (Q2_K,
+# Q3_K, IQ4_XS up to 48 in a row) or 12: (512, 18944, 3584) 16.2, one flush, tiles
+# whole and split, 128 tokens wide; (250, 16384, 12544) 24.5, two flushes, summed by
+# a fixup launch or 6 workgroups' last; (40, 33000, 12544) and (20, 33000, 12544)
+# 24.7, 64 and 32 tokens wide, ragged rows.
+@pytest.mark.parametrize("M,N,K", [(512, 18944, 3584), (250, 16384, 12544), (40, 33000, 12544), (20, 33000, 12544)])
+@pytest.mark.parametrize("qt", LOW)
+def test_gemm_long_chains(tc, dev, oracle, qt, M, N, K):
+    """Where a workgroup holds more superblocks of a tile than one chain of fp32
+    sums, the sums that it flushes to memory and takes back; the bounds derived at
+    test_gemm_low_bit_mfma and test_gemm_fp32_activations_mfma."""
+    rng = np.random.default_rng(M + N + K + qt)
+    w = even_blocks(qt, rng, N, K)
+    x = gaussian(rng, (M, K))
+    got = tc.gemm(qt, to_dev(w, dev), to_dev(x, dev), N, K).cpu().numpy()
+    rows, toks = tile_edges(N, 256, 16, rng)[::3], tile_edges(M, 32, 4, rng)
+    wr = w.reshape(N, -1)[rows]
+    ref = oracle_matmul_par(oracle, qt, wr, x[toks], len(rows), K)
+    wa = np.abs(oracle.dequant(qt, wr, len(rows), K).reshape(len(rows), K).astype(np.float64))
+    if qt in (IQ4_NL, Q5_0, IQ2_XS):
+        bound = 2 * (K // 32 + 12) * 2.0**-24 * (np.abs(x[toks].astype(np.float64)) @ wa.T)
+    else:
+        qs, d, _ = oracle.quantize_q8k(x[toks].ravel())
+        xa = np.abs(qs.reshape(-1, 256).astype(np.float64) * d.reshape(-1, 1)).reshape(len(toks), K)
+        bound = 2 * (K // 256 + 10) * 2.0**-24 * (xa @ wa.T)
+    worst = (np.abs(got[np.ix_(toks, rows)] - ref) / bound).max()
+    assert worst <= 1, f"{NAMES[qt]} M={M} N={N} K={K}: worst err/bound {worst:.3g}"
+    assert np.isfinite(got).all()
 
 
 @pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ4_XS])

@@ -31,9 +31,9 @@ inline bool ok(int rc) {
 inline bool int8GemmAvailable() { return tc_available() != 0; }
 
 /// out[seqLen][rows] = x[seqLen][cols] @ W[rows][cols]^T on the int8 matrix
-/// cores (Q4_K, Q5_K, Q6_K, Q8_0, IQ3_XXS, IQ3_S, IQ2_S) or the exact batched
-/// mat-vec (Q2_K, Q3_K, IQ2_XS, IQ4_XS, IQ4_NL, Q5_0)
-/// (reference int8Gemm, Int8Gemm.hpp:57-59).
+/// cores (Q4_K, Q5_K, Q6_K, Q8_0, IQ3_XXS, IQ3_S, IQ2_S; from 9 tokens Q2_K,
+/// Q3_K, IQ4_XS), on the bf16 ones from 9 tokens IQ2_XS, IQ4_NL, Q5_0, else as
+/// int8Gemv (reference int8Gemm, Int8Gemm.hpp:57-59).
 inline bool int8Gemm(int type, const void *w, const float *x, float *out, uint32_t seqLen, uint32_t rows,
                      uint32_t cols, uint32_t blocksPerRow, void *stream) {
     return detail::ok(tc_gemm(type, w, x, out, seqLen, rows, cols, blocksPerRow, stream));
@@ -52,7 +52,7 @@ inline bool int8Gemv(int type, const void *w, const float *x, float *out, uint32
     return detail::ok(tc_gemv(type, w, x, out, seqLen, rows, cols, stream));
 }
 
-/// Pre-size the activation scratch (reference int8GemvReserve, Int8Gemm.hpp:82).
+/// Pre-size the scratch (reference int8GemvReserve, Int8Gemm.hpp:82).
 inline void int8GemvReserve(uint32_t cols, uint32_t seqLen) { (void)tc_gemv_reserve(cols, seqLen); }
 
 /// Enable/disable the Q8_0 GEMM path (reference int8GemmSetQ8Enabled,

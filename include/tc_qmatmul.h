@@ -52,8 +52,8 @@ int tc_available(void);
 
 /* Decode mat-vec, seq_len 1..8: out[s][r] = x[s] . W[r]. Several tokens whose
  * activations do not fit one launch of the decode kernel go through tc_gemm's
- * kernels where those are faster and as accurate (under stream capture: where the scratch is in place, by
- * tc_gemv_reserve or an earlier call; else by the decode kernel).
+ * kernels where those are faster and as accurate; under stream capture only
+ * where the scratch is in place, by tc_gemv_reserve or an earlier call.
  * Replaces tinycoder::gpu::int8Gemv (include/Int8Gemm.hpp:77-78,
  * src/cpp/core/cuda/gemm/GemmDispatch.cu:788). cols % 256 == 0. */
 int tc_gemv(int type, const void *w, const float *x, float *out, uint32_t seq_len, uint32_t rows,
@@ -144,13 +144,14 @@ int tc_quantize_act(int type, const float *x, uint32_t seq_len, uint32_t cols, i
  * reference's parity hooks GPUModel::debugQ8KBlocks / debugQ8_0Blocks,
  * include/GPUCompute.hpp:399-460, as a free function over a whole matrix):
  * isums[seq_len][rows][nblk][k], k = 8 sub-block sums for Q4_K, else 1
- * (nblk = cols/32 for Q8_0). The same kernel as tc_gemv computes them. */
+ * (nblk = cols/32 for Q8_0). The decode kernel computes them, which serves
+ * tc_gemv's single tokens and most calls of several. */
 int tc_block_isums(int type, const void *w, const float *x, int32_t *isums, uint32_t seq_len,
                    uint32_t rows, uint32_t cols, void *stream);
 
 /* Weight encoder: fp32 [rows][cols] -> raw GGUF blocks of `type`. Q4_K is the
  * reference's own quantizer (src/cpp/core/GGMLQuantize.cpp:47, bit-exact);
- * Q8_0 / Q6_K / IQ3_XXS are this library's encoders (the reference has none).
+ * the other types' are this library's encoders (the reference has none).
  * Replaces GGMLQuantize::quantizeQ4KBlock (include/GGMLQuantize.hpp:56). */
 int tc_encode(int type, const float *x, void *out, uint32_t rows, uint32_t cols, void *stream);
 
@@ -164,7 +165,7 @@ size_t tc_row_bytes(int type, uint32_t cols);
  * wg, wu: [n_experts][ff][hidden]; wd: [n_experts][hidden][ff] (Q4_K blocks).
  * ids int32 [seq_len][top_k], wts fp32 [seq_len][top_k], x [seq_len][hidden],
  * out [seq_len][hidden]; all device pointers.
- * From tc_moe_set_gemm_min_tokens tokens on (default 160; the prefill case
+ * From tc_moe_set_gemm_min_tokens tokens on (default 40; the prefill case
  * of the reference's moeBatchExperts, MoeBatch.cu:37-197) the pairs are
  * sorted by expert on the device and each matrix runs as ONE grouped int8
  * MFMA GEMM over all experts; below it, one mat-vec per (token, rank) pair. */

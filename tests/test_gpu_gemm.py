@@ -1,7 +1,7 @@
-"""GPU parity tests for the prefill GEMM (tc_gemm, int8 MFMA for Q4_K / Q5_K /
-Q6_K / IQ3_XXS / IQ3_S / IQ2_S / Q8_0, the exact batched mat-vec path (IQ2_XS
-on fp32 x) for Q2_K / Q3_K / IQ4_XS / IQ4_NL / Q5_0 / IQ2_XS), through the
-C-ABI.
+"""GPU parity tests for the prefill GEMM (tc_gemm: int8 MFMA for Q4_K / Q5_K /
+Q6_K / IQ3_XXS / IQ3_S / IQ2_S / Q8_0 and, from 9 tokens, Q2_K / Q3_K / IQ4_XS;
+bf16 MFMA on the pieces of fp32 x for IQ4_NL / Q5_0 / IQ2_XS; the decode kernel
+over groups of tokens for the calls of those six that it keeps), through the C-ABI.
 
 Bar: fp32 outputs within 1e-3 relative / 1e-4 absolute of the oracle (the C
 restatement of the reference CPU kernels, itself bit-exact with the compiled
@@ -369,6 +369,9 @@ for qt in (tc_hip.Q2_K, tc_hip.Q3_K, tc_hip.IQ4_XS, tc_hip.IQ4_NL, tc_hip.Q5_0, 
 
 @pytest.mark.parametrize("qt", [Q2_K, Q3_K, IQ2_XS, IQ4_XS, IQ4_NL, Q5_0])
 def test_gemm_exact_batched_types(tc, dev, oracle, qt):
+    """The types that the reference's GEMM leaves to its exact batched path, on
+    the matrix cores here (test_gemm_captured_without_scratch runs the decode
+    kernel over groups of tokens)."""
     rng = np.random.default_rng(5 + qt)
     M, N, K = 21, 80, 512
     w = enc_weights(oracle, qt, rng, N, K)

@@ -93,11 +93,8 @@ __device__ __forceinline__ uint32_t quant4_sum(float4 v, float iscale, int *sum)
 }
 
 // One 256-element Q8_K block by one full wave, lane values already loaded
-// (lane l holds elements 4l..4l+3). Writes qs[0..255], *d and bsums[0..15],
-// and with dg the 32-wide sums s_p = bsums[2p] + bsums[2p + 1] as two exact
-// bf16 pieces: dg[p] = 128 * (s_p >> 7), dg[8 + p] = s_p & 127.
-// A quantized block in the wave's registers: lane l's values 4l .. 4l + 3, the
-// sum of its group of 16, and the block's d.
+// (lane l holds elements 4l..4l+3), left in the wave's registers: lane l's
+// values 4l .. 4l + 3, the sum of its group of 16, and the block's d.
 struct Q8KLane {
     uint32_t packed;
     int s16;
@@ -126,6 +123,9 @@ __device__ __forceinline__ void q8k_pieces(int s16, uint16_t &hi, uint16_t &lo) 
     lo = uint16_t(__builtin_bit_cast(uint32_t, float(s32 & 127)) >> 16);
 }
 
+// The same written out: qs[0..255], *d and bsums[0..15], and with dg the 32-wide
+// sums s_p = bsums[2p] + bsums[2p + 1] as two exact bf16 pieces: dg[p] = 128 *
+// (s_p >> 7), dg[8 + p] = s_p & 127.
 __device__ __forceinline__ void quant_q8k_block_wave_v(float4 v, int8_t *qs, float *d, int16_t *bsums,
                                                        uint16_t *dg = nullptr) {
     const uint32_t lane = threadIdx.x & 63;

@@ -70,19 +70,19 @@ hipError_t launch_moe_combine(const float *y, const float *wts, float *out, uint
 hipError_t launch_gemv_jobs(int type, uint32_t S, const GemvJob *jobs, uint32_t njobs, int num_cu,
                             hipStream_t st);
 
-// Largest token count per mat-vec launch for this width (LDS budget).
 // Weight bytes one mat-vec launch streams over the jobs (both matrices of a pair).
 uint64_t jobs_weight_bytes(int type, const GemvJob *jobs, uint32_t njobs);
 // Largest S*cols a mat-vec launch over `weight_bytes` quantizes in-kernel
 // without loading x after the weights; wider inputs are quantized by a
 // separate launch first.
 uint32_t gemv_fused_quant_limit(int type, uint64_t weight_bytes);
+// Largest token count per mat-vec launch for this width (LDS budget; 0: none).
 uint32_t gemv_max_tokens(int type, uint32_t cols);
 
 // Prefill GEMM (int8 MFMA): out[M][N] = W x^T with the activations already
 // quantized (launch_quant_act over M tokens, block-major) and the weights
 // converted in the MFMA lanes' registers, once per token tile of up to 128
-// tokens (tc_prefill.hip; Q4_K, Q5_K, Q6_K, Q8_0, IQ3_XXS, IQ3_S, IQ2_S).
+// tokens (tc_prefill.hip; Q2_K to Q6_K, Q8_0, IQ3_XXS, IQ3_S, IQ2_S, IQ4_XS).
 // Stream-K over one workgroup per CU. Q4_K, Q5_K and Q8_0 need the
 // activations' scale data (act.dg); every type prefill_workspace_bytes() of scratch
 // whose first prefill_counter_words() 32-bit words are zero when the launch

@@ -4,7 +4,8 @@
 // cores (v_mfma_f32_32x32x16_bf16).
 //
 // x = h + m + l exactly, three bf16 pieces of 8 significant bits each (the
-// sign and the 24 bits of an fp32), split once per call by k_split_bf16; the
+// sign and the 24 bits of an fp32; of |x| below 2^-103 what lies under the
+// smallest normal number may be lost), split once per call by k_split_bf16; the
 // integer weights (|q| <= 127) are exact in bf16, so every product q * piece
 // is exact and only the sums round, in fp32 as in the decode kernel. Per
 // 32-block (16 weights for IQ2_XS, whose scales are per 16) six (three) MFMAs
